@@ -131,6 +131,11 @@ int mnb_plan_device_bytes(const mnb_plan *plan, size_t *bytes);
  *    exact route serves larger M 16 rows at a time), its split activation
  *    image and fp32 partial sums (none where the fragment-ordered M <= 4
  *    GEMV serves them);
+ *  - where the automatic path is the exact GEMM (accuracy_level 1 above 16
+ *    rows; K not a multiple of 64), for the at most 2048 rows of one of its
+ *    launches: their split activation image (4 bytes per value, 6 where K is
+ *    not a multiple of 64), the exponents and the partial sums of its K runs
+ *    (less workspace: launches of fewer rows, then the kernels below);
  *  - for 1 or 2 rows too long for one workgroup per 64-row group (K > 16384
  *    at M = 1, K > 8192 at M = 2; plain plans), the fragment-ordered GEMV
  *    with K split into S segments: (S - 1)*M*N*4 bytes of partial sums;
@@ -160,16 +165,19 @@ int mnb_workspace_bytes(const mnb_plan *plan, int64_t M, size_t *bytes);
  * (unset, this library's default) and 2-4 take the GEMM, whose 11-bit
  * activations meet what levels 2-4 permit. M > 16 with K an odd multiple
  * of 32, which the GEMM kernels do not take, runs path 4 at every level;
- * K not a multiple of 32 runs the generic kernel (path 3). The launch is
- * asynchronous on `stream`. */
+ * K not a multiple of 32 runs path 3. With the workspace, path 4 multiplies
+ * whole groups of 16 rows (every row where K is not a multiple of 64) in the
+ * exact GEMM, whose groups are bit-identical to the decode kernels', and the
+ * automatic path 3 takes the exact GEMM (all 24 bits of A) where it is
+ * faster than the generic kernel. The launch is asynchronous on `stream`. */
 int mnb_run(const mnb_plan *plan, int64_t M, const float *dA, float *dY, void *dWorkspace,
             size_t workspace_bytes, void *stream);
 
 /* Same as mnb_run with the kernel chosen by the caller (whatever the plan's
  * accuracy_level): path 0 = automatic, 1 = decode GEMV (any M <= 16),
  * 2 = MFMA GEMM (any M; the kernel picked by shape), 3 = generic fallback
- * (any shape; slow, for cross-checks), 4 = the decode kernels over
- * consecutive groups of 16 rows (any M; the exact route of accuracy_level 1),
+ * (any shape; slow, for cross-checks), 4 = the exact route of accuracy_level 1
+ * (any M; groups of 16 rows: the exact GEMM, the decode kernels),
  * 5 = the MFMA GEMM's prefill kernel over the plan's fragment-ordered weight
  * copy (any M; MNB_ERR_UNSUPPORTED when the plan holds none: K % 64 != 0,
  * N % 4 != 0, block_size < 32 or N >= 2^22). */

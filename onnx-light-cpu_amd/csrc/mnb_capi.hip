@@ -211,6 +211,26 @@ int DerivePlanConstants(mnb_plan *p) {
       }
       FillView(p);
     }
+  } else if (mnb::ExactRaggedLayoutWanted(p->view)) {
+    // K that 64-k tiles do not divide: the exact GEMM's layout alone.
+    size_t zd_bytes = 0;
+    const size_t bp_bytes = mnb::ExactRaggedLayoutBytes(p->view);
+    const size_t sd_bytes = mnb::DecodeFragScaleBytes(p->view, &zd_bytes);
+    e = hipMalloc(reinterpret_cast<void **>(&p->dBp), bp_bytes);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&p->dSd), sd_bytes);
+    if (e == hipSuccess && zd_bytes > 0) e = hipMalloc(reinterpret_cast<void **>(&p->dZd), zd_bytes);
+    if (e != hipSuccess) {
+      SetLastError("hipMalloc", e);
+      return MNB_ERR_ALLOC;
+    }
+    e = mnb::LaunchExactRaggedRelayout(p->view, p->dBp, nullptr);
+    if (e == hipSuccess) e = mnb::LaunchDecodeFragRelayout(p->view, p->dSd, p->dZd, nullptr);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+      SetLastError("exact re-layout", e);
+      return MNB_ERR_HIP;
+    }
+    FillView(p);
   }
   // Compact plan: where every automatic route reads only the re-laid copies,
   // a plan that owns its weights drops the original layout (about 2.07x the
@@ -553,9 +573,11 @@ int mnb_plan_device_bytes(const mnb_plan *plan, size_t *bytes) {
   if (plan->owns && plan->dB != nullptr)
     total += N * static_cast<size_t>(row_bytes) + N * static_cast<size_t>(nb) * sizeof(float) +
              (plan->dZ != nullptr ? N * static_cast<size_t>(zp_row_bytes) : 0);
-  if (plan->dBp != nullptr) {
+  if (plan->dBp != nullptr && plan->dSp != nullptr) {
     size_t sp = 0;
     total += mnb::PrefillLayoutBytes(plan->view, &sp) + sp;
+  } else if (plan->dBp != nullptr) {
+    total += mnb::ExactRaggedLayoutBytes(plan->view);
   }
   if (plan->dSd != nullptr) {
     size_t zd = 0;
@@ -706,6 +728,61 @@ static bool GateUpFusedInGemv(const mnb_plan *plan, int64_t M, int path, bool rm
   return plan->gate_up && path == 1 && mnb::GemvFragPreferred(plan->view, M, rms);
 }
 
+// accuracy_level is ONNX Runtime's MatMulNBits attribute: the lowest accuracy
+// at which A may enter the computation (0 unset, 1 fp32, 2 fp16, 3 bf16,
+// 4 int8). Level 1 asks for fp32 activations, so its rows never take the
+// fp16 GEMM: above 16 rows they go through the exact-product kernels (path
+// 4). Levels 0 (unset: the library's default), 2, 3 and 4 take the fp16 GEMM
+// above 16 rows, whose activations keep an 11-bit significand with per-row
+// range scaling: at least the accuracy levels 2-4 permit. Every level runs
+// the exact decode kernels up to 16 rows.
+static bool Fp32ActivationsOnly(const mnb_plan *plan) { return plan->desc.accuracy_level == 1; }
+
+// Rows of the first exact-GEMM launch for M rows of an automatic (or path 4)
+// run whose selected path is `path`, with work_bytes of workspace; 0 where the
+// other kernels of that path serve.
+// - 64-k plans (path 4): whole groups of 16 rows from 32 rows up, bit-identical
+//   to the decode kernels' groups, which serve the remaining rows.
+// - K that 64-k tiles do not divide, all rows: path 4 (K a multiple of 32,
+//   above 16 rows), and path 3 where GenericKernel's one wavefront per column
+//   takes longer than this route's three launches: its time grows by about
+//   4.5 ns per M K, and with N past the 8192 wavefronts the chip holds
+//   (graph replay, us, GenericKernel against this: K = 300, N = 4000 M = 4
+//   10.7 / 11.4, M = 8 19.1 / 11.4; K = 1003, N = 4000 M = 1 8.5 / 13.2,
+//   M = 2 14.5 / 13.2; K = 1003, N = 12000 M = 1 17.8 / 13.3; K = 2500,
+//   N = 500 M = 1 13.2 / 13.5; K = 2500, N = 5001 M = 333 6350 / 45).
+// A launch takes at most kExactMaxRows rows (its image is then at most 1.5
+// KiB per unit and row), fewer where the workspace is smaller.
+constexpr int64_t kExactMaxRows = 2048;
+
+static bool ExactBeatsGeneric(const mnb_plan *plan, int64_t M) {
+  const int64_t mk = M * plan->view.K;
+  return mk >= 2400 || mk * plan->view.N >= 8000000;
+}
+
+static int64_t ExactRows(const mnb_plan *plan, int64_t M, int path, size_t work_bytes) {
+  const bool ragged = (plan->view.K % 64) != 0;
+  const int64_t step = ragged ? 1 : 16;
+  if (path != 4 && !(path == 3 && ragged)) return 0;
+  if (path == 3 ? !ExactBeatsGeneric(plan, M) : M < (ragged ? 17 : 32)) return 0;
+  int64_t rows = std::min(M, kExactMaxRows) / step * step;
+  while (mnb::ExactSupports(plan->view, rows)) {
+    if (GateUpScratchBytes(plan, rows) + mnb::ExactWorkspaceBytes(plan->view, rows) <= work_bytes)
+      return rows;
+    if (rows <= 32) break;
+    rows = (rows / 2 + 31) / 32 * 32;
+  }
+  return 0;
+}
+
+// Workspace of the exact GEMM's first launch for M rows on `path` (0 where it
+// does not serve): the rest of the rows fit it or take smaller launches.
+static size_t ExactNeed(const mnb_plan *plan, int64_t M, int path) {
+  const int64_t rows = ExactRows(plan, M, path, ~size_t{0});
+  return rows == 0 ? 0 : mnb::ExactWorkspaceBytes(plan->view, rows);
+}
+
+static int SelectPath(const mnb_plan *plan, int64_t M, const float *dA);
 
 int mnb_workspace_bytes(const mnb_plan *plan, int64_t M, size_t *bytes) {
   if (plan == nullptr || bytes == nullptr) return MNB_ERR_NULL_POINTER;
@@ -715,7 +792,8 @@ int mnb_workspace_bytes(const mnb_plan *plan, int64_t M, size_t *bytes) {
   // and the MFMA decode kernel (split-K partial sums).
   // A gate/up plan adds the scratch sum in front of either.
   // The exact route (path 4) runs the decode kernels over groups of at most
-  // 16 rows, one after another in the same workspace.
+  // 16 rows, one after another in the same workspace; the exact GEMM's
+  // launches, where the automatic path takes it, likewise.
   // Decode launches served by the fragment-ordered GEMV need none. The
   // decode kernel of a fused RMSNorm input (mnb_run_rmsnorm passes this
   // size on) may differ from the plain one: the size covers both.
@@ -723,20 +801,11 @@ int mnb_workspace_bytes(const mnb_plan *plan, int64_t M, size_t *bytes) {
   if (M > 0 && mnb::GemmSupports(plan->view, M)) need = mnb::GemmWorkspaceBytes(plan->view, M);
   const int64_t md = std::min<int64_t>(M, kExactGroupRows);
   if (md > 0) need = std::max({need, DecodeNeed(plan, md), DecodeNeed(plan, md, true)});
+  if (M > 0 && (Fp32ActivationsOnly(plan) || (plan->view.K % 64) != 0))
+    need = std::max(need, ExactNeed(plan, M, SelectPath(plan, M, nullptr)));
   *bytes = need + GateUpScratchBytes(plan, M);
   return MNB_OK;
 }
-
-
-// accuracy_level is ONNX Runtime's MatMulNBits attribute: the lowest accuracy
-// at which A may enter the computation (0 unset, 1 fp32, 2 fp16, 3 bf16,
-// 4 int8). Level 1 asks for fp32 activations, so its rows never take the
-// fp16 GEMM: above 16 rows they go through the exact-product decode kernels,
-// 16 rows at a time (path 4). Levels 0 (unset: the library's default), 2, 3
-// and 4 take the fp16 GEMM above 16 rows, whose activations keep an 11-bit
-// significand with per-row range scaling: at least the accuracy levels 2-4
-// permit. Every level runs the exact decode kernels up to 16 rows.
-static bool Fp32ActivationsOnly(const mnb_plan *plan) { return plan->desc.accuracy_level == 1; }
 
 static bool ExactGroupsSupported(const mnb_plan *plan, bool a_aligned) {
   return a_aligned && DecodeSupported(plan, kExactGroupRows);
@@ -752,6 +821,14 @@ static int SelectPath(const mnb_plan *plan, int64_t M, const float *dA) {
   return ExactGroupsSupported(plan, a_aligned) ? 4 : 3;
 }
 
+// Bytes of the largest exact-GEMM launch of these rows that fits the
+// no-allocation scratch.
+static size_t ExactFitBytes(const mnb_plan *plan, int64_t M, int path) {
+  const int64_t rows = ExactRows(plan, M, path, kScratchBytes);
+  return rows == 0 ? 0
+                   : GateUpScratchBytes(plan, rows) + mnb::ExactWorkspaceBytes(plan->view, rows);
+}
+
 // Workspace the automatic path (mnb_run) takes for M rows of dA: the chosen
 // kernel's own, plus a gate/up plan's scratch sum where its epilogue does not
 // apply the activation (the exact route: per group of 16 rows).
@@ -763,9 +840,10 @@ static size_t AutoWorkspaceBytes(const mnb_plan *plan, int64_t M, const float *d
   case 2: return mnb::GemmWorkspaceBytes(plan->view, M) + GateUpScratchBytes(plan, M);
   case 4: {
     const int64_t md = std::min<int64_t>(M, kExactGroupRows);
-    return DecodeNeed(plan, md) + GateUpScratchBytes(plan, md);
+    return std::max(DecodeNeed(plan, md) + GateUpScratchBytes(plan, md),
+                    ExactFitBytes(plan, M, path));
   }
-  default: return GateUpScratchBytes(plan, M);
+  default: return std::max(GateUpScratchBytes(plan, M), ExactFitBytes(plan, M, path));
   }
 }
 
@@ -774,6 +852,28 @@ int mnb_select_path(const mnb_plan *plan, int64_t M, int *path) {
   if (M < 0) return MNB_ERR_BAD_SHAPE;
   // Paths are chosen for a 16-byte-aligned activation buffer, as hipMalloc returns.
   *path = SelectPath(plan, M, nullptr);
+  return MNB_OK;
+}
+
+// One exact-GEMM launch of `rows` rows (ExactRows): on a gate/up plan the
+// scratch sum, then the kernel's own workspace.
+static int RunExact(const mnb_plan *plan, int64_t rows, const float *dA, const float *dBias,
+                    float *dY, void *dWorkspace, void *stream) {
+  int cur = -1;
+  if (hipGetDevice(&cur) != hipSuccess || cur != plan->device) {
+    std::snprintf(g_last_error, sizeof(g_last_error), "plan lives on device %d, current is %d",
+                  plan->device, cur);
+    return MNB_ERR_NO_DEVICE;
+  }
+  const size_t scratch = GateUpScratchBytes(plan, rows);
+  float *Ys = plan->gate_up ? static_cast<float *>(dWorkspace) : dY;
+  const hipError_t e = mnb::LaunchExact(
+      plan->view, rows, dA, Ys, static_cast<char *>(dWorkspace) + scratch,
+      reinterpret_cast<hipStream_t>(stream), plan->gate_up ? dY : nullptr, dBias);
+  if (e != hipSuccess) {
+    SetLastError("kernel launch", e);
+    return MNB_ERR_HIP;
+  }
   return MNB_OK;
 }
 
@@ -789,24 +889,37 @@ static int RunImpl(const mnb_plan *plan, int64_t M, const float *dA, const float
   if (dA == nullptr || dY == nullptr) return MNB_ERR_NULL_POINTER;
   if (path < 0 || path > 5) return MNB_ERR_UNSUPPORTED;
   const bool a_aligned = (reinterpret_cast<uintptr_t>(dA) % 16) == 0;
-  if (path == 0) path = SelectPath(plan, M, dA);
+  const bool automatic = path == 0;
+  if (automatic) path = SelectPath(plan, M, dA);
   if (path == 1 && !(a_aligned && DecodeSupported(plan, M))) return MNB_ERR_UNSUPPORTED;
   if (path == 2 && !(a_aligned && mnb::GemmSupports(plan->view, M))) return MNB_ERR_UNSUPPORTED;
   if (path == 4 && !ExactGroupsSupported(plan, a_aligned)) return MNB_ERR_UNSUPPORTED;
   if (path == 5 && !(a_aligned && mnb::PrefillSupports(plan->view, M))) return MNB_ERR_UNSUPPORTED;
   if (plan->gate_up && dBias != nullptr) return MNB_ERR_UNSUPPORTED;
-  if (path == 4) {
-    // The decode kernels over consecutive groups of rows, in stream order on
-    // the one workspace (each group's launches finish reading it before the
-    // next group's start writing it).
+  if (path == 4 || (path == 3 && automatic)) {
+    // The exact GEMM over as many rows as it takes, then (path 4) the decode
+    // kernels over consecutive groups of rows, all in stream order on the one
+    // workspace (each launch finishes reading it before the next writes it).
     const int64_t K = plan->view.K, cols = plan->gate_up ? plan->view.N / 2 : plan->view.N;
-    for (int64_t m0 = 0; m0 < M; m0 += kExactGroupRows) {
-      const int64_t mg = std::min(kExactGroupRows, M - m0);
-      const int st = RunImpl(plan, mg, dA + m0 * K, dBias, dY + m0 * cols, dWorkspace,
-                             workspace_bytes, stream, 1, nullptr, 0.0f);
-      if (st != MNB_OK) return st;
+    int64_t m0 = 0;
+    if (dWorkspace != nullptr && (reinterpret_cast<uintptr_t>(dWorkspace) % 16) == 0) {
+      while (const int64_t rows = ExactRows(plan, M - m0, path, workspace_bytes)) {
+        const int st = RunExact(plan, rows, dA + m0 * K, dBias, dY + m0 * cols, dWorkspace, stream);
+        if (st != MNB_OK) return st;
+        m0 += rows;
+      }
     }
-    return MNB_OK;
+    if (m0 == M) return MNB_OK;
+    const int64_t group = path == 4 ? kExactGroupRows : M - m0;
+    if (path == 4 || m0 > 0) {
+      for (; m0 < M; m0 += group) {
+        const int64_t mg = std::min(group, M - m0);
+        const int st = RunImpl(plan, mg, dA + m0 * K, dBias, dY + m0 * cols, dWorkspace,
+                               workspace_bytes, stream, path == 4 ? 1 : 3, nullptr, 0.0f);
+        if (st != MNB_OK) return st;
+      }
+      return MNB_OK;
+    }
   }
   // A gate/up plan's runs start with the scratch sum; the path's own
   // workspace follows it.
@@ -990,7 +1103,9 @@ const char *mnb_kernel_name(const mnb_plan *plan, int64_t M, size_t workspace_by
     if (workspace_bytes < scratch) return "";
     work_bytes -= scratch;
   }
-  switch (SelectPath(plan, M, reinterpret_cast<const float *>(uintptr_t{256}))) {
+  const int path = SelectPath(plan, M, reinterpret_cast<const float *>(uintptr_t{256}));
+  if (ExactRows(plan, M, path, workspace_bytes) > 0) return "ExactKernel";
+  switch (path) {
   case 1:
     switch (PickDecodeKernel(plan, M, work, work_bytes)) {
     case kDecM1: return "GemvM1Kernel";

@@ -69,7 +69,6 @@ namespace df {
 using namespace dec;
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -85,35 +84,6 @@ constexpr int kStepBytes = kTerms * 1024;  // image bytes per 32-k step (16 toke
 template <int TOKS>
 constexpr int StepBytesT() { return TOKS == 16 ? kStepBytes : 1024; }
 constexpr int kMaxSqUnits = 64;            // RMSNorm input: K <= 64 units (16384)
-
-__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
-  const half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-// 8 nibbles (k order) of one word -> q - zp as fp16 in [0,4,1,5,2,6,3,7]
-// order, exact: (w & 0x000F000F) | 0x6400.. is the fp16 pair 1024 + q of
-// nibbles 0 | 4 (ulp 1 at 1024), (w & 0x00F000F0) | 0x5400.. the pair 64 + q
-// of nibbles 1 | 5 (ulp 1/16 at 64); the same of w >> 8 gives nibbles 2 | 6
-// and 3 | 7. neg_lo / neg_hi are the fp16 pairs -(1024 + zp) / -(64 + zp).
-// The masks sit in VGPRs (v_and_or_b32 takes no literal on gfx9).
-struct Masks {
-  uint32_t lo, hi, e1024, e64;
-};
-__device__ __forceinline__ Masks MakeMasks() {
-  Masks c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
-  return c;
-}
-__device__ __forceinline__ half8 DecodeQ(uint32_t w, uint32_t neg_lo, uint32_t neg_hi,
-                                         const Masks &c) {
-  const uint32_t w8 = w >> 8;
-  const uint4 r = make_uint4(PkAddF16((w & c.lo) | c.e1024, neg_lo),
-                             PkAddF16((w & c.hi) | c.e64, neg_hi),
-                             PkAddF16((w8 & c.lo) | c.e1024, neg_lo),
-                             PkAddF16((w8 & c.hi) | c.e64, neg_hi));
-  return __builtin_bit_cast(half8, r);
-}
 
 // One wavefront (a workgroup of 64 threads) per unit u and pair of tokens:
 // lane (t, ch) of workgroup (u, pair) takes the 8 values k = 256 u + 8 ch ..
@@ -581,8 +551,7 @@ hipError_t LaunchZp(const WeightView &w, int64_t M, const Work &wk, float *Y, fl
 } // namespace df
 
 bool DecodeFragLayoutWanted(const WeightView &w) {
-  return (w.K % 32) == 0 && w.block_size >= 32 &&
-         (w.block_size & (w.block_size - 1)) == 0 && w.K <= (int64_t{1} << 24) &&
+  return w.block_size >= 32 && (w.block_size & (w.block_size - 1)) == 0 && w.K <= (int64_t{1} << 24) &&
          w.N < (int64_t{1} << 22) && w.nb * 256 < (int64_t{1} << 31);
 }
 
@@ -601,13 +570,19 @@ hipError_t LaunchDecodeFragRelayout(const WeightView &w, float *Sd, uint32_t *Zd
 
 bool DecodeFragSupports(const WeightView &w, int64_t M) {
   return M >= 2 && M <= 16 && w.Bp != nullptr && w.Sd != nullptr &&
-         (!w.has_zp || w.Zd != nullptr) && DecodeFragLayoutWanted(w) &&
+         (!w.has_zp || w.Zd != nullptr) && (w.K % 64) == 0 && DecodeFragLayoutWanted(w) &&
          M * w.K * 4 + 4096 < (int64_t{1} << 31) && M * w.N * 4 < (int64_t{1} << 31) &&
          (w.K / 32) * df::kStepBytes < (int64_t{1} << 31);
 }
 
 bool DecodeFragTakesRms(const WeightView &w) {
   return w.K <= df::kMaxSqUnits * df::kUnitK && (w.K % df::kUnitK) == 0;
+}
+
+void DecodeFragRuns(const WeightView &w, int *run_units, int *range_units) {
+  const df::Shape sh = df::PickShape(w, 0, 0);
+  *run_units = sh.wpg * sh.units_per_wave;
+  *range_units = sh.units_per_wave;
 }
 
 size_t DecodeFragWorkspaceBytes(const WeightView &w, int64_t M, int wpg, int units_per_wave) {

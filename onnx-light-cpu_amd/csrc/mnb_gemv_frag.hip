@@ -733,7 +733,7 @@ bool GemvFragSegSupports(const WeightView &w, int64_t M) {
   // 48 Mi elements, where they beat the fp32-FMA GEMV.
   if (M < 1 || M > 4 || w.Bp == nullptr || w.Sd == nullptr || (w.has_zp && w.Zd == nullptr) ||
       w.block_size < 32 || w.block_size > 256 || (w.block_size & (w.block_size - 1)) != 0 ||
-      (w.K % 32) != 0)
+      (w.K % 64) != 0)
     return false;
   const int64_t kn = w.K * w.N;
   const bool long_narrow = w.K >= 5120 && kn <= (int64_t{192} << 20);

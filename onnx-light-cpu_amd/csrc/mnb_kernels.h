@@ -216,6 +216,27 @@ hipError_t LaunchDecodeFrag(const WeightView &w, int64_t M, const float *A, floa
                             hipStream_t s, float *H = nullptr, int wpg = 0,
                             int units_per_wave = 0, const float *bias = nullptr,
                             const float *gamma = nullptr, float eps = 0.0f);
+// The K structure of its launch: units (256 k) per run (one workgroup) and per
+// range (one wavefront). Sums go range by range, then run by run.
+void DecodeFragRuns(const WeightView &w, int *run_units, int *range_units);
+
+// Many rows with the activations split into fp16 terms, on the
+// fragment-ordered copy (mnb_exact.hip). 64-k plans: whole groups of 16 rows
+// (M % 16 == 0) with two terms, each group bit-identical to LaunchDecodeFrag
+// at 16 rows. Plans of any other K (the ragged layout): any M, three terms
+// (every bit of A). `work` holds ExactWorkspaceBytes(w, M): the operand image
+// (M padded to 32 rows, 2 bytes per term and value of whole units), the units'
+// exponents and the partial sums of runs 1... bias not with H.
+bool ExactSupports(const WeightView &w, int64_t M);
+size_t ExactWorkspaceBytes(const WeightView &w, int64_t M);
+hipError_t LaunchExact(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
+                       hipStream_t s, float *H = nullptr, const float *bias = nullptr);
+// The ragged layout: Bp for K % 64 != 0, the records of whole 64-k tiles with
+// zero weights past the row's bytes (with Sd / Zd as for DecodeFragKernel).
+// No other kernel reads it: they take K % 64 == 0.
+bool ExactRaggedLayoutWanted(const WeightView &w);
+size_t ExactRaggedLayoutBytes(const WeightView &w);
+hipError_t LaunchExactRaggedRelayout(const WeightView &w, uint8_t *Bp, hipStream_t s);
 // Y += P[0] + ... + P[parts - 1] over mn elements, in that order (then the
 // gate/up activation into H when H is not null).
 hipError_t LaunchSumPartials(float *Y, const float *P, int64_t mn, int parts, float *H,

@@ -1,0 +1,147 @@
+"""GPU: the exact-activation GEMM (mnb_exact.hip) at the sizes where it can go
+wrong: row tiles of 16 and 32 and their remainders, column tiles of 256, K
+that ends inside a block, a word, a 64-k tile or a 256-k unit, one and several
+K runs, launches of fewer rows than the call (a small workspace).
+
+K not a multiple of 64 (three activation terms, every bit of A) against the
+fp64 oracle at the decode bound 1e-5; accuracy_level 1 (two terms) bit for bit
+against the decode kernels' groups of 16 rows. Every case prints its shape and
+kernel before touching the GPU.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+def _plan(pkg, K, N, bs, zp, seed, level=0):
+    p = pkg.workloads.Projection("exact", K, N, bs, zp)
+    B, S, Z = pkg.workloads.make_weights(p, seed)
+    return pkg.MatMulNBits(K, N, 4, bs, accuracy_level=level).prepare(B, S, Z), B, S, Z
+
+
+@pytest.mark.parametrize("K,N,bs,zp,M", [
+    (2401, 1, 32, True, 1),        # one column; K one past a step
+    (65, 257, 32, False, 40),      # second 64-k tile of one value; one column past the tile
+    (255, 255, 64, True, 16),      # a unit less one value; a full row tile of 16
+    (257, 256, 128, True, 17),     # a second unit of one value; one row past the tile
+    (1000, 300, 256, False, 31),   # blocks of a whole unit
+    (1000, 300, 512, True, 33),    # blocks longer than a unit
+    (5000, 70, 32, False, 64),     # many runs on one column tile
+    (3100, 9000, 64, True, 300),   # every run in one workgroup
+    (4128, 130, 128, True, 50),    # K an odd multiple of 32 (path 4)
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_ragged_k(pkg, orc, cuda, K, N, bs, zp, M, bias):
+    import torch
+    op, B, S, Z = _plan(pkg, K, N, bs, zp, K + N + M)
+    A = pkg.workloads.make_activations(M, K, 1.0, M + 1)
+    b = np.random.default_rng(N).standard_normal(N).astype(np.float32)
+    print(f"case exact ragged K={K} N={N} bs={bs} zp={zp} M={M} kernel={op.kernel_name(M)}",
+          flush=True)
+    assert op.kernel_name(M) == "ExactKernel"
+    buf = torch.full((M * N + 8,), float("nan"), device=cuda)
+    out = buf[4:4 + M * N].view(M, N)
+    op(torch.from_numpy(A).to(cuda), out=out, bias=torch.from_numpy(b).to(cuda) if bias else None)
+    Y = out.cpu().numpy()
+    assert torch.isnan(buf[:4]).all() and torch.isnan(buf[4 + M * N:]).all()
+    op.release()
+    y64 = orc.matmul_nbits_f64(A, B, S, Z, K, N, bs) + (b.astype(np.float64) if bias else 0.0)
+    assert orc.normwise_max_error(Y, y64) <= TOL
+
+
+@pytest.mark.parametrize("K,N,bs,zp,M", [
+    (512, 64, 32, True, 32),       # one row tile, one unit per wavefront and run
+    (1088, 260, 64, False, 48),    # a last unit of one tile; 1.5 row tiles
+    (4096, 6144, 32, True, 80),    # four runs, partial sums
+    (4096, 14336, 256, True, 96),  # one run of eight ranges
+    (14336, 4096, 128, True, 512),  # four runs in one workgroup
+    (1024, 128, 128, True, 2064),  # two launches (2048 + 16 rows)
+])
+def test_level_1_groups_are_the_decode_kernels(pkg, cuda, K, N, bs, zp, M):
+    import torch
+    op, *_ = _plan(pkg, K, N, bs, zp, K + M, level=1)
+    A = torch.from_numpy(pkg.workloads.make_activations(M, K, 1.0, M + 2)).to(cuda)
+    print(f"case exact level 1 K={K} N={N} bs={bs} M={M} kernel={op.kernel_name(M)}", flush=True)
+    assert op.kernel_name(M) == "ExactKernel"
+    Y = op(A)
+    for m0 in sorted({0, 16, M // 32 * 16, M - 16}):
+        ref = op(A[m0:m0 + 16].contiguous(), path=pkg.PATH_GEMV)
+        assert torch.equal(Y[m0:m0 + 16], ref), m0
+    op.release()
+
+
+def test_non_finite_rows(pkg, orc, cuda):
+    """+inf, -inf and NaN keep the reference's kinds and stay in their row,
+    also next to the values past K that a tile holds."""
+    import torch
+    K, N, bs, M = 1003, 70, 32, 20
+    op, B, S, Z = _plan(pkg, K, N, bs, True, 5)
+    A = pkg.workloads.make_activations(M, K, 1.0, 6)
+    clean = op(torch.from_numpy(A).to(cuda)).cpu().numpy()
+    bad = A.copy()
+    bad[3, 37], bad[7, K - 1], bad[17, 5] = np.inf, -np.inf, np.nan
+    print(f"case exact non-finite K={K} kernel={op.kernel_name(M)}", flush=True)
+    Y = op(torch.from_numpy(bad).to(cuda)).cpu().numpy()
+    op.release()
+    rows = [3, 7, 17]
+    keep = [m for m in range(M) if m not in rows]
+    np.testing.assert_array_equal(Y[keep], clean[keep])
+    ref = orc.matmul_nbits_ref_f32(bad[rows], B, S, Z, K, N, bs)
+    for kind in (np.isposinf, np.isneginf, np.isnan):
+        np.testing.assert_array_equal(kind(Y[rows]), kind(ref))
+
+
+@pytest.mark.parametrize("K,level", [(1000, 0), (1024, 1)])
+def test_small_workspaces(pkg, orc, cuda, K, level):
+    """Less workspace than asked for: launches of fewer rows (every row the
+    same bits), then the kernels without the image."""
+    import torch
+    N, bs, M = 192, 64, 200
+    op, B, S, Z = _plan(pkg, K, N, bs, False, 9, level=level)
+    A = pkg.workloads.make_activations(M, K, 1.0, 10)
+    dA = torch.from_numpy(A).to(cuda)
+    y64 = orc.matmul_nbits_f64(A, B, S, Z, K, N, bs)
+    L = pkg.library()
+    need = op.workspace_bytes(M)
+    work = torch.empty(need, dtype=torch.uint8, device=cuda)
+    for nbytes in (need, need // 2, need // 5, 0):
+        Y = torch.full((M, N), float("nan"), device=cuda)
+        print(f"case exact workspace K={K} {nbytes} of {need}: {op.kernel_name(M, nbytes)}", flush=True)
+        st = L.mnb_run(op._plan, M, ctypes.c_void_p(dA.data_ptr()), ctypes.c_void_p(Y.data_ptr()),
+                       ctypes.c_void_p(work.data_ptr()) if nbytes else None, nbytes,
+                       ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert st == 0
+        assert orc.normwise_max_error(Y.cpu().numpy(), y64) <= TOL
+    op.release()
+
+
+def test_gate_up_and_graph(pkg, orc, cuda):
+    """The gate/up activation behind one and several runs, and a captured call
+    replayed on changed activations."""
+    import torch
+    K, I, bs, M = 1000, 100, 32, 40
+    p = pkg.workloads.Projection("gu", K, I, bs, True)
+    W = [pkg.workloads.make_weights(p, s) for s in (61, 62)]
+    gu = pkg.GateUpSiLU(K, I, 4, bs).prepare(*W[0], *W[1])
+    A = pkg.workloads.make_activations(M, K, 1.0, 63)
+    dA = torch.from_numpy(A).to(cuda)
+    out = torch.empty(M, I, device=cuda)
+    print(f"case exact gate/up K={K} I={I} kernel={gu.kernel_name(M)}", flush=True)
+    gu(dA, out=out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gu(dA, out=out)
+    for seed in (63, 64, 65):
+        A = pkg.workloads.make_activations(M, K, 1.0, seed)
+        dA.copy_(torch.from_numpy(A))
+        out.fill_(float("nan"))
+        g.replay()
+        h64 = orc.gate_up_silu_f64(A, *W[0], *W[1], K, I, bs)
+        assert orc.normwise_max_error(out.cpu().numpy(), h64) <= 4 * TOL
+    gu.release()
