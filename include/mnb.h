@@ -123,7 +123,8 @@ int mnb_plan_device_bytes(const mnb_plan *plan, size_t *bytes);
  * rows, whichever path serves them (0 when none): the larger of
  *  - the prefill GEMM's: A scaled per row by a power of two and rounded to
  *    fp16 in its tile layout, ceil(M/128)*128*K*2 bytes, the rows' exponents
- *    (ceil(M/128)*128 int32, rounded up to 256 bytes), then, when the GEMM
+ *    (ceil(M/128)*128 int32, rounded up to 256 bytes; up to 64 rows that many
+ *    words for each started 512 of K), then, when the GEMM
  *    splits K into S > 1 parts, (S - 1)*M*N*4 bytes of fp32 partial sums
  *    (S <= 16, chosen from the shape);
  *  - where an MFMA decode kernel with a workspace serves min(M, 16) rows

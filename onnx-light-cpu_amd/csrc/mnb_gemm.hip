@@ -36,7 +36,7 @@
 //    Tile order is XCD-aware: workgroup b runs on XCD b % 8; when the M tiles
 //    split evenly over the 8 XCDs, XCD x gets a contiguous band of M tiles with
 //    all their N tiles, so each XCD's L2 holds one slab of A.
-#include "mnb_kernels.h"
+#include "mnb_gemm_common.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -45,14 +45,10 @@
 namespace mnb {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
+using namespace gemm;
 
 constexpr int kMaxBM = 128;  // largest tile height; the workspace pads M to it
 constexpr int kBN = 128;
-constexpr int kBK = 64;
-constexpr int kUnits = kBK / 8;             // 16-byte units per LDS row
 constexpr int kBUnits = kBN * kUnits;       // units per B tile (16 KiB)
 constexpr int kAStages = 3;
 // Output tiles are BM x 128 with BM in {32, 64, 128}; A tiles BM x 64 fp16.
@@ -60,68 +56,6 @@ template <int BM>
 constexpr int AUnits() { return BM * kUnits; }  // units per A tile
 template <int BM>
 constexpr size_t LdsBytes() { return (kAStages * AUnits<BM>() + 2 * kBUnits) * 16; }  // <= 80 KiB
-
-__device__ __forceinline__ int Swz(int row, int unit) {
-  return row * kUnits + (unit ^ ((row >> 1) & 7));
-}
-
-__device__ __forceinline__ uint32_t PackHalf2(float lo, float hi) {
-  const half2v h = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
-  return __builtin_bit_cast(uint32_t, h);
-}
-
-__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
-  const half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-__device__ __forceinline__ uint32_t PkMulF16(uint32_t a, uint32_t b) {
-  const half2v r = __builtin_bit_cast(half2v, a) * __builtin_bit_cast(half2v, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-// Per-thread constants of the dequantization, held in VGPRs (an empty asm
-// hides their values from the compiler): VOP3 instructions on gfx9 take no
-// literal, so with the masks as literals (w & m) | c costs two instructions
-// instead of one v_and_or_b32.
-struct DequantConsts {
-  uint32_t lo, hi, e1024, e64;  // 0x000F000F, 0x00F000F0, fp16 pairs 1024.0, 64.0
-};
-__device__ __forceinline__ DequantConsts MakeDequantConsts() {
-  DequantConsts c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
-  return c;
-}
-
-// Per (row, k-tile) operands of DequantWord: -(1024 + zp) and -(64 + zp)
-// (exact in fp16) and the block scale in fp16.
-struct DequantRow {
-  uint32_t neg_lo, neg_hi, s;
-};
-__device__ __forceinline__ DequantRow MakeDequantRow(float s, uint32_t zp) {
-  const float z = static_cast<float>(zp);
-  return DequantRow{PackHalf2(-(1024.f + z), -(1024.f + z)), PackHalf2(-(64.f + z), -(64.f + z)),
-                    PackHalf2(s, s)};
-}
-
-// One packed word of 8 nibbles (k order) -> 8 fp16 weights in [0,4,1,5,2,6,3,7]
-// order, with no per-nibble shift: in fp16, 1024.0 (0x6400) has an ulp of 1
-// and 64.0 (0x5400) an ulp of 1/16, so (w & 0x000F000F) | 0x6400.. is the
-// pair 1024 + q of nibbles 0 | 4 and (w & 0x00F000F0) | 0x5400.. the pair
-// 64 + q of nibbles 1 | 5, both exact; the same of w >> 8 gives nibbles
-// 2 | 6 and 3 | 7. Adding -(1024 + zp) or -(64 + zp) leaves q - zp exactly,
-// and one multiply by the fp16 scale rounds the weight once. Per word: one
-// shift, four v_and_or_b32, four packed adds and four packed multiplies.
-__device__ __forceinline__ uint4 DequantWord(uint32_t w, const DequantRow &r,
-                                             const DequantConsts &c) {
-  const uint32_t w8 = w >> 8;
-  const uint32_t h0 = (w & c.lo) | c.e1024;   // nibbles 0 | 4: 1024 + q
-  const uint32_t h1 = (w & c.hi) | c.e64;     // nibbles 1 | 5: 64 + q
-  const uint32_t h2 = (w8 & c.lo) | c.e1024;  // nibbles 2 | 6
-  const uint32_t h3 = (w8 & c.hi) | c.e64;    // nibbles 3 | 7
-  return make_uint4(PkMulF16(PkAddF16(h0, r.neg_lo), r.s), PkMulF16(PkAddF16(h1, r.neg_hi), r.s),
-                    PkMulF16(PkAddF16(h2, r.neg_lo), r.s), PkMulF16(PkAddF16(h3, r.neg_hi), r.s));
-}
 
 // Largest value over the 256 threads of a workgroup (4 wavefronts); every
 // thread gets it. `red` holds 4 floats of LDS.
@@ -233,11 +167,93 @@ __global__ __launch_bounds__(256) void ConvertAKernel(const float *__restrict__ 
   }
 }
 
-// s_waitcnt vmcnt(N) with the other counters left free (gfx9 encoding: vmcnt
-// in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <int N>
-__device__ __forceinline__ void WaitVm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+// StreamKernel's conversion of A: one workgroup of 8 wavefronts per (chunk of
+// kChunkK k, group of 16 rows), wavefront w its steps 2 w and 2 w + 1, lane l
+// 8 k of row l & 15 per step. Each row's chunk is scaled by 2^f, f =
+// RangeExponent of the chunk's largest magnitude (StreamKernel's wavefronts
+// stay inside one chunk and undo f in their sums), rounded to fp16 as
+// ConvertAKernel does and written as 1 KiB operand records, the lanes
+// contiguous: no row-wide reduction, whole cache lines per store. With gamma
+// (RMSNorm folded in) the values are x * gamma and sq receives each row's sum
+// of x^2 over the chunk, from which StreamKernel forms 1 / rms.
+constexpr int kChunkK = 512;
+template <bool RMS>
+__global__ __launch_bounds__(512) void ConvertChunkKernel(const float *__restrict__ A,
+                                                          uint4 *__restrict__ img,
+                                                          int *__restrict__ exps,
+                                                          float *__restrict__ sq,
+                                                          const float *__restrict__ gamma, int M,
+                                                          int K, int chunks, int rows_padded) {
+  __shared__ float red[8][16], reds[RMS ? 8 : 1][16];
+  const int ch = static_cast<int>(blockIdx.x) % chunks;
+  const int mt = static_cast<int>(blockIdx.x) / chunks;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15;
+  const int T = K / 32;
+  const int rows = min(16, M - 16 * mt);
+  const int bytes = rows * K * 4;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(A + static_cast<size_t>(16 * mt) * K), 0, bytes, 0x00020000);
+  floatx4 x[2][2], gm[2][2];
+  float amax = 0.0f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    // rows past M and steps past K read beyond the buffer: zeros
+    const int s = ch * (kChunkK / 32) + 2 * wave + h;
+    const int vo = r < rows && s < T ? (r * K + 32 * s + 8 * (lane >> 4)) * 4 : bytes;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      x[h][p] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra, vo + 16 * p, 0, 0));
+      if constexpr (RMS)
+        gm[h][p] = reinterpret_cast<const floatx4 *>(gamma + 32 * min(s, T - 1) + 8 * (lane >> 4))[p];
+    }
+  }
+  if constexpr (RMS) {
+    float q = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) q += x[h][p][v] * x[h][p][v];
+        x[h][p] *= gm[h][p];
+      }
+    q += Xor16(q);
+    q += __shfl_xor(q, 32, 64);
+    if (lane < 16) reds[wave][lane] = q;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) amax = fmaxf(amax, fabsf(x[h][p][v]));
+  amax = fmaxf(amax, Xor16(amax));
+  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+  if (lane < 16) red[wave][lane] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) amax = fmaxf(amax, red[w][r]);
+  const int f = RangeExponent(amax, kRowExpTarget);
+  if (threadIdx.x < 16) {
+    exps[ch * rows_padded + 16 * mt + lane] = f;
+    if constexpr (RMS) {
+      float q = 0.0f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) q += reds[w][lane];
+      sq[ch * rows_padded + 16 * mt + lane] = q;
+    }
+  }
+  auto sc = [f](float v) { return __builtin_amdgcn_ldexpf(v, f); };
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int s = ch * (kChunkK / 32) + 2 * wave + h;
+    const floatx4 a = x[h][0], b = x[h][1];
+    if (s < T)
+      img[(static_cast<size_t>(mt) * T + s) * 64 + lane] =
+          make_uint4(PackHalf2(sc(a[0]), sc(b[0])), PackHalf2(sc(a[1]), sc(b[1])),
+                     PackHalf2(sc(a[2]), sc(b[2])), PackHalf2(sc(a[3]), sc(b[3])));
+  }
 }
 
 // One k-tile of B for this thread: 32 nibbles of one weight row (one
@@ -667,8 +683,11 @@ inline size_t AImageBytes(const WeightView &w, int64_t M) {
   return static_cast<size_t>(PaddedRows(M)) * static_cast<size_t>(w.K) * 2;
 }
 
-inline size_t RowExpBytes(int64_t M) {
-  return (static_cast<size_t>(PaddedRows(M)) * 4 + 255) / 256 * 256;
+inline size_t RowExpBytes(const WeightView &w, int64_t M) {
+  // StreamKernel (at most 64 rows): an exponent and a sum of squares per row
+  // and chunk of K
+  const size_t chunks = M <= 64 ? static_cast<size_t>((w.K + kChunkK - 1) / kChunkK) : 1;
+  return (static_cast<size_t>(PaddedRows(M)) * 4 * chunks + 255) / 256 * 256;
 }
 
 inline size_t PartialBytes(const WeightView &w, int64_t M, const Shape &sh) {
@@ -711,7 +730,7 @@ hipError_t LaunchBM(const WeightView &w, int64_t M, const float *A, float *Y, vo
   uint4 *Ah = static_cast<uint4 *>(work);
   int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *partials = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                              RowExpBytes(M));
+                                              RowExpBytes(w, M));
   hipError_t e = gamma != nullptr
                      ? LaunchConvertA<BM, true>(w, M, A, Ah, row_exp, s, gamma, eps)
                      : LaunchConvertA<BM, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
@@ -754,8 +773,8 @@ inline Shape PickShape(const WeightView &w, int64_t M) {
 // word (8 nibbles, original order) of weight row 64g + 16j + (l & 15) at k =
 // 32s + 8(l >> 4): exactly lane l's MFMA operand for the 16 rows of slice j.
 // The 256-byte record Sp[g][b][c][j] holds, per quantization block b, the
-// fp16 scale (times the row's 2^e) in the low half and the zero point in the
-// high half, for row 64g + 16j + c. Rows past N are zero (scale 0). One record
+// fp16 scale (times the row's 2^e) in the low half, the zero point in byte 2
+// and 16 times it in byte 3, for row 64g + 16j + c. Rows past N are zero (scale 0). One record
 // per block, not per step: every step of a block reads the same record.
 //
 // A workgroup of 8 wavefronts (two per SIMD, one workgroup per CU) computes a
@@ -797,22 +816,6 @@ constexpr int kPOps1 = kPAU / kPThreads + 1;          // wavefronts 4-7 (no scal
 // plain stores serve it better (c4 and c5 o at M = 512, 4 splits: 37.1 ->
 // 35.4 and 38.0 -> 36.3 us per call; qkv at M = 256 33.2 -> 32.2).
 constexpr int kStoreNT = 2;
-
-// (scale fp16 | zp << 16) -> the operands of DequantWord.
-template <bool HAS_ZP>
-__device__ __forceinline__ DequantRow RowFromSz(uint32_t w) {
-  DequantRow r;
-  r.s = __builtin_amdgcn_perm(w, w, 0x01000100u);  // the fp16 scale in both halves
-  if constexpr (HAS_ZP) {
-    const uint32_t z = w >> 16;
-    r.neg_lo = 0xE400E400u + z * 0x00010001u;  // fp16 -(1024 + z): ulp 1 at 1024
-    r.neg_hi = 0xD400D400u + z * 0x00100010u;  // fp16 -(64 + z): ulp 1/16 at 64
-  } else {
-    r.neg_lo = 0xE408E408u;  // -(1024 + 8)
-    r.neg_hi = 0xD480D480u;  // -(64 + 8)
-  }
-  return r;
-}
 
 template <bool HAS_ZP, bool BS32>
 __global__ __launch_bounds__(kPThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
@@ -1081,16 +1084,21 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
 // segment. Per step a wavefront loads the group's 1 KiB weight record and
 // 256-byte scale record (the PrefillKernel layouts), dequantizes the four
 // words exactly as PrefillKernel does (DequantWord on the fp16 scale times
-// 2^e_n), reads TG activation fragments of the fp16 image ConvertAKernel
-// wrote (BM = 64 tiling, rows scaled by 2^f_m, rows past M zero) and issues
+// 2^e_n), reads TG activation fragments of the fp16 image ConvertChunkKernel
+// wrote (rows past M zero) and issues
 // 4 TG v_mfma_f32_16x16x32_f16 into TG x 4 fp32 tiles. The operands are
-// those of the prefill GEMM, so the product is the same up to the order of
-// the fp32 sums. Loads stream through a rolling window of WIN steps in
+// those of the prefill GEMM (a chunk's exponent instead of the row's), so the
+// product is the same up to the order of the fp32 sums. Loads stream through a rolling window of WIN steps in
 // registers (multiply the oldest, issue the one WIN further on), with no
 // branch around any load. The wavefronts' tiles meet in LDS and are added
 // in wavefront order; segment 0 writes Y (adding the bias or applying the
 // gate/up activation when K is not split), segment s > 0 its partial sum,
 // added in segment order by SplitReduceKernel.
+//
+// G = 2 takes two column groups per workgroup, each activation fragment loaded
+// once for both: with many groups the loads of the activations (TG KiB per
+// step beside 1.25 KiB of weights, from the L2) bound the kernel (K = 4096,
+// N = 28672, 448 groups: M = 48 / 64 30.4 / 34.0 -> 27.3 / 29.8 us).
 constexpr int kSGroupRows = 64;
 
 //
@@ -1103,34 +1111,37 @@ constexpr int kSGroupRows = 64;
 // the wavefronts' tiles meet. A finer exponent than the row's, so the
 // operands are ConvertAKernel's except where those fall into fp16
 // subnormals.
-template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT>
+template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
 __global__ __launch_bounds__(512) void StreamKernel(
     const uint4 *__restrict__ Ah, const float *__restrict__ A, const uint8_t *__restrict__ Bp,
     const uint8_t *__restrict__ Sp, float *__restrict__ Y, float *__restrict__ partials,
     float *__restrict__ H, const int *__restrict__ row_exp, const int *__restrict__ col_exp,
-    const float *__restrict__ bias, int M, int N, int K, int log2_bs, int segs, int wpg) {
-  extern __shared__ floatx4 sred[];  // [wave][tg * 4 + j][lane]
+    const float *__restrict__ bias, const float *__restrict__ sq, float eps, int M, int N, int K,
+    int log2_bs, int segs, int wpg) {
+  extern __shared__ floatx4 sred[];  // [wave][2 tg + (j & 1)][lane], j / 2 one half
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int g = static_cast<int>(blockIdx.x) / segs;
-  const int seg = static_cast<int>(blockIdx.x) - g * segs;
+  const int g = static_cast<int>(blockIdx.x) / segs * G;  // first group
+  const int seg = static_cast<int>(blockIdx.x) % segs;
   const int T = K / 32;
   const int s0 = (seg * wpg + wave) * SPW;  // first step of this wavefront
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t *>(Bp + static_cast<size_t>(g) * T * 1024), 0, T * 1024, 0x00020000);
+  __amdgpu_buffer_rsrc_t rb[G], rs[G];
   const int nb = (K + (1 << log2_bs) - 1) >> log2_bs;
   const int sb_shift = log2_bs - 5;  // 32-k steps per block, log2
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t *>(Sp + static_cast<size_t>(g) * nb * 256), 0, nb * 256, 0x00020000);
+#pragma unroll
+  for (int x = 0; x < G; ++x) {  // a G past the last group reads zero weights (padded records)
+    rb[x] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(Bp + static_cast<size_t>(g + x) * T * 1024), 0, T * 1024, 0x00020000);
+    rs[x] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(Sp + static_cast<size_t>(g + x) * nb * 256), 0, nb * 256, 0x00020000);
+  }
+  // Lane l's activation fragment tg of step s: 16 bytes of the 1 KiB record
+  // (tg, s), contiguous over the lanes. (In the prefill kernel's swizzled rows
+  // every four lanes of such a load fall into four cache lines, and the L1's
+  // one line per cycle bounded the kernel: K = 4096, N = 28672 at M = 48 / 64 35.4 / 41.6 ->
+  // 29.7 / 33.9 us.)
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint4 *>(Ah), 0, (K / kBK) * AUnits<kSGroupRows>() * 16, 0x00020000);
-  // Lane l's activation fragment tg of step s: row 16 tg + (l & 15), unit
-  // 4 (s & 1) + (l >> 4) of k-tile s / 2 (the PrefillKernel operand order).
-  int aoff[TG][2];
-#pragma unroll
-  for (int tg = 0; tg < TG; ++tg)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) aoff[tg][h] = Swz(16 * tg + (lane & 15), 4 * h + (lane >> 4)) * 16;
+      const_cast<uint4 *>(Ah), 0, TG * T * 1024, 0x00020000);
 
   typedef uint32_t u32x4e __attribute__((ext_vector_type(4)));
   typedef float f32x4e __attribute__((ext_vector_type(4)));
@@ -1153,50 +1164,66 @@ __global__ __launch_bounds__(512) void StreamKernel(
     }
   }
   struct Slot {
-    u32x4e w, sz;
+    u32x4e w[G], sz[G];
     half8 a[CVT ? 1 : TG];
   };
   Slot ring[WIN];
   auto issue = [&](int i) __attribute__((always_inline)) {
     Slot &sl = ring[i % WIN];
     const int s = s0 + i;
-    sl.w = __builtin_bit_cast(u32x4e, __builtin_amdgcn_raw_buffer_load_b128(rb, s * 1024 + 16 * lane, 0, 2));
-    sl.sz = __builtin_bit_cast(u32x4e, __builtin_amdgcn_raw_buffer_load_b128(
-                                           rs, (s >> sb_shift) * 256 + 16 * (lane & 15), 0, 0));
+#pragma unroll
+    for (int x = 0; x < G; ++x) {
+      sl.w[x] = __builtin_bit_cast(
+          u32x4e, __builtin_amdgcn_raw_buffer_load_b128(rb[x], s * 1024 + 16 * lane, 0, 2));
+      sl.sz[x] = __builtin_bit_cast(u32x4e, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rs[x], (s >> sb_shift) * 256 + 16 * (lane & 15), 0, 0));
+    }
     if constexpr (!CVT) {
-      const int kt = s >> 1;
 #pragma unroll
       for (int tg = 0; tg < TG; ++tg)
         sl.a[tg] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 ra, kt * (AUnits<kSGroupRows>() * 16) + aoff[tg][s & 1], 0, 0));
+                                                 ra, (tg * T + s) * 1024 + 16 * lane, 0, 0));
     }
   };
 #pragma unroll
   for (int i = 0; i < WIN && i < SPW; ++i) issue(i);
-  // The epilogue's exponents and bias for the fragments x = wave, wave + wpg,
-  // ... this wavefront finishes (at most 4: wpg >= 4), loaded behind the
-  // first weights so their latency hides under the main loop.
-  constexpr int kMaxItems = (TG * 4 + 3) / 4;
-  int er[kMaxItems];
+  // The epilogue finishes, group by group and half by half (kHalf fragments
+  // (tg, j) with j / 2 == half), fragments x = wave, wave + wpg, ... of each
+  // (wpg >= 4). Their exponents and bias are loaded behind the first weights so
+  // that their latency hides under the main loop (with two groups, whose
+  // registers they would take, in the epilogue).
+  constexpr int kHalf = 2 * TG;
+  constexpr int kHalfItems = (kHalf + 3) / 4;
+  constexpr int kMaxItems = 2 * G * kHalfItems;
+  constexpr bool kPreload = G == 1;
   int4 ec[kMaxItems];
   float4 bv[kMaxItems];
-#pragma unroll
-  for (int it = 0; it < kMaxItems; ++it) {
-    const int x = min(wave + it * wpg, TG * 4 - 1);
-    const int m = min(16 * (x >> 2) + (lane & 15), M - 1);
-    const int nc = min(kSGroupRows * g + 16 * (x & 3) + 4 * (lane >> 4), N - 4);
-    er[it] = CVT ? 0 : row_exp[m];
+  auto item_col = [&](int it) {
+    const int x = min(wave + it % kHalfItems * wpg, kHalf - 1), ph = it / kHalfItems;
+    return kSGroupRows * (g + ph / 2) + 16 * (2 * (ph & 1) + (x & 1)) + 4 * (lane >> 4);
+  };
+  auto item_load = [&](int it) __attribute__((always_inline)) {
+    const int nc = min(item_col(it), N - 4);
     ec[it] = *reinterpret_cast<const int4 *>(col_exp + nc);
     bv[it] = bias != nullptr ? make_float4(bias[nc], bias[nc + 1], bias[nc + 2], bias[nc + 3])
                              : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  if constexpr (kPreload) {
+#pragma unroll
+    for (int it = 0; it < kMaxItems; ++it) item_load(it);
   }
   __builtin_amdgcn_sched_barrier(0);
 
   // CVT: each row's exponent over this wavefront's k range (the row's values
   // sit in lanes r, r + 16, r + 32, r + 48), then the fp16 fragments.
   half8 af[CVT ? SPW : 1][CVT ? TG : 1];
-  int fw[CVT ? TG : 1];
-  if constexpr (CVT) {
+  int fw[TG];
+  if constexpr (!CVT) {
+    // the chunk's (a wavefront past K reads the last chunk's and adds nothing)
+    const int ch = min(s0 / (kChunkK / 32), (T - 1) / (kChunkK / 32));
+#pragma unroll
+    for (int tg = 0; tg < TG; ++tg) fw[tg] = row_exp[ch * 16 * TG + 16 * tg + (lane & 15)];
+  } else {
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg) {
       float amax = 0.0f;
@@ -1222,89 +1249,111 @@ __global__ __launch_bounds__(512) void StreamKernel(
   }
 
   const DequantConsts dq = MakeDequantConsts();
-  floatx4 acc[TG][4];
+  floatx4 acc[G][TG][4];
 #pragma unroll
-  for (int tg = 0; tg < TG; ++tg)
+  for (int x = 0; x < G; ++x)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[tg][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int tg = 0; tg < TG; ++tg)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[x][tg][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < SPW; ++i) {
     Slot &sl = ring[i % WIN];
-    __asm__ volatile("" : "+v"(sl.w), "+v"(sl.sz));
-    const uint32_t wv[4] = {sl.w[0], sl.w[1], sl.w[2], sl.w[3]};
-    const uint32_t zv[4] = {sl.sz[0], sl.sz[1], sl.sz[2], sl.sz[3]};
-    half8 bf[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      bf[j] = __builtin_bit_cast(half8, DequantWord(wv[j], RowFromSz<HAS_ZP>(zv[j]), dq));
+    for (int x = 0; x < G; ++x) __asm__ volatile("" : "+v"(sl.w[x]), "+v"(sl.sz[x]));
 #pragma unroll
-    for (int tg = 0; tg < TG; ++tg) {
-      half8 a;
-      if constexpr (CVT)
-        a = af[i][tg];
-      else
-        a = sl.a[tg];
+    for (int x = 0; x < G; ++x) {
+      half8 bf[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        acc[tg][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j], a, acc[tg][j], 0, 0, 0);
+        bf[j] = __builtin_bit_cast(half8, DequantWord(sl.w[x][j], RowFromSz<HAS_ZP>(sl.sz[x][j]), dq));
+#pragma unroll
+      for (int tg = 0; tg < TG; ++tg) {
+        half8 a;
+        if constexpr (CVT)
+          a = af[i][tg];
+        else
+          a = sl.a[tg];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[x][tg][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[j], a, acc[x][tg][j], 0, 0, 0);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     if (i + WIN < SPW) issue(i + WIN);
     __builtin_amdgcn_sched_barrier(0);
   }
-
-  // The wavefronts' tiles meet in LDS; wavefront w then finishes the
-  // fragments x = (tg, j) = w, w + wpg, ..., adding the wavefronts' tiles in
-  // wavefront order. Lane l holds row 16 tg + (l & 15) and the 4 columns
-  // 64 g + 16 j + 4 (l >> 4) .. + 3. A wavefront past K (the end of a
-  // shorter last segment) ran on loads beyond the weights' buffers (zeros)
-  // and activations past its rows: it adds nothing.
-  const bool past_k = s0 >= T;
+  // RMSNorm input: each row's 1 / rms from the chunks' sums of squares.
+  float inv[TG];
 #pragma unroll
-  for (int tg = 0; tg < TG; ++tg)
+  for (int tg = 0; tg < TG; ++tg) inv[tg] = 1.0f;
+  if (sq != nullptr) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      floatx4 t = acc[tg][j];
-      if constexpr (CVT) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) t[q] = __builtin_amdgcn_ldexpf(t[q], -fw[tg]);
-      }
-      sred[(wave * TG * 4 + tg * 4 + j) * 64 + lane] = past_k ? floatx4{0.f, 0.f, 0.f, 0.f} : t;
+    for (int tg = 0; tg < TG; ++tg) {
+      float q = 0.0f;
+      for (int ch = 0; ch * kChunkK < K; ++ch) q += sq[ch * 16 * TG + 16 * tg + (lane & 15)];
+      inv[tg] = 1.0f / sqrtf(q / static_cast<float>(K) + eps);
     }
-  __syncthreads();
+  }
+
+  // The wavefronts' tiles meet in LDS, half the fragments (j = 0, 1, then 2,
+  // 3) at a time so that two workgroups fit a CU; wavefront w finishes the
+  // half's fragments x = 2 tg + (j & 1) = w, w + wpg, ..., adding the
+  // wavefronts' tiles in wavefront order. Lane l holds row 16 tg + (l & 15)
+  // and the 4 columns 64 g + 16 j + 4 (l >> 4) .. + 3. A wavefront past K
+  // (the end of a shorter last segment) ran on loads beyond the weights'
+  // buffers (zeros) and activations past its rows: it adds nothing.
+  const bool past_k = s0 >= T;
   float *out = seg == 0 ? Y : partials + static_cast<size_t>(seg - 1) * M * N;
 #pragma unroll
-  for (int it = 0; it < kMaxItems; ++it) {
-    const int x = wave + it * wpg;
-    if (x >= TG * 4) break;
-    floatx4 sum = sred[x * 64 + lane];
-    for (int w = 1; w < wpg; ++w) sum += sred[(w * TG * 4 + x) * 64 + lane];
-    const int tg = x >> 2, j = x & 3;
-    const int m = 16 * tg + (lane & 15);
-    const int n = kSGroupRows * g + 16 * j + 4 * (lane >> 4);
-    const int ecv[4] = {ec[it].x, ec[it].y, ec[it].z, ec[it].w};
-    floatx4 v;
+  for (int ph = 0; ph < 2 * G; ++ph) {  // (group, half)
+    const int half = ph & 1;
+    if (ph > 0) __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_ldexpf(sum[q], -((CVT ? 0 : er[it]) + ecv[q]));
-    const bool ok = m < M && n < N;
-    if (H != nullptr) {
-      // gate/up pairs (columns n, n + 1 and n + 2, n + 3): H columns n / 2, n / 2 + 1
-      const int half_n = N >> 1;
-      const auto hr = __builtin_amdgcn_make_buffer_rsrc(H, 0, M * half_n * 4, 0x00020000);
-      typedef unsigned int u32x2 __attribute__((vector_size(8)));
-      const u32x2 hv = {__float_as_uint(SiluMul(v[0], v[1])), __float_as_uint(SiluMul(v[2], v[3]))};
-      __builtin_amdgcn_raw_buffer_store_b64(hv, hr, ok ? (m * half_n + (n >> 1)) * 4 : M * half_n * 4, 0, 0);
-    } else {
-      if (bias != nullptr) {
-        v[0] += bv[it].x;
-        v[1] += bv[it].y;
-        v[2] += bv[it].z;
-        v[3] += bv[it].w;
+    for (int tg = 0; tg < TG; ++tg)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) {
+        floatx4 t = acc[ph / 2][tg][2 * half + jj];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) t[q] = __builtin_amdgcn_ldexpf(t[q], -fw[tg]) * inv[tg];
+        sred[(wave * kHalf + tg * 2 + jj) * 64 + lane] = past_k ? floatx4{0.f, 0.f, 0.f, 0.f} : t;
       }
-      const auto yr = __builtin_amdgcn_make_buffer_rsrc(out, 0, M * N * 4, 0x00020000);
-      typedef unsigned int u32x4 __attribute__((vector_size(16)));
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), yr,
-                                             ok ? (m * N + n) * 4 : M * N * 4, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int hi = 0; hi < kHalfItems; ++hi) {
+      const int x = wave + hi * wpg;
+      if (x >= kHalf) break;
+      const int it = ph * kHalfItems + hi;
+      if constexpr (!kPreload) item_load(it);
+      floatx4 sum = sred[x * 64 + lane];
+      for (int w = 1; w < wpg; ++w) sum += sred[(w * kHalf + x) * 64 + lane];
+      const int m = 16 * (x >> 1) + (lane & 15);
+      const int n = item_col(it);
+      const int ecv[4] = {ec[it].x, ec[it].y, ec[it].z, ec[it].w};
+      floatx4 v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_ldexpf(sum[q], -ecv[q]);
+      const bool ok = m < M && n < N;
+      if (H != nullptr) {
+        // gate/up pairs (columns n, n + 1 and n + 2, n + 3): H columns n / 2, n / 2 + 1
+        const int half_n = N >> 1;
+        const auto hr = __builtin_amdgcn_make_buffer_rsrc(H, 0, M * half_n * 4, 0x00020000);
+        typedef unsigned int u32x2 __attribute__((vector_size(8)));
+        const u32x2 hv = {__float_as_uint(SiluMul(v[0], v[1])), __float_as_uint(SiluMul(v[2], v[3]))};
+        __builtin_amdgcn_raw_buffer_store_b64(
+            hv, hr, ok ? (m * half_n + (n >> 1)) * 4 : M * half_n * 4, 0, 0);
+      } else {
+        if (bias != nullptr) {
+          v[0] += bv[it].x;
+          v[1] += bv[it].y;
+          v[2] += bv[it].z;
+          v[3] += bv[it].w;
+        }
+        const auto yr = __builtin_amdgcn_make_buffer_rsrc(out, 0, M * N * 4, 0x00020000);
+        typedef unsigned int u32x4 __attribute__((vector_size(16)));
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), yr,
+                                               ok ? (m * N + n) * 4 : M * N * 4, 0, 0);
+      }
     }
   }
 }
@@ -1312,54 +1361,54 @@ __global__ __launch_bounds__(512) void StreamKernel(
 struct StreamShape {
   int segs, wpg, spw;
   bool ragged = false;  // a shorter last segment
+  int groups = 1;       // 64-row groups per workgroup
 };
+// Steps in flight with two groups per wavefront: 16 (w, sz) + 4 TG VGPRs each
+// beside 32 TG accumulators.
+template <int TG>
+constexpr int WinG2() { return TG == 2 ? 4 : TG == 3 ? 3 : 2; }
 
-// K segments, wavefronts per workgroup and steps per wavefront (segs * wpg *
-// spw = K / 32): the fewest segments whose workgroups cover 85% of the CUs
-// (else the most that leave a workgroup at least 16 steps), then 8
-// wavefronts before 4 and the longest spw in {16, 8, 4}. Step counts with no
-// such division (K = 11008: 344 steps = 8 x 43) take segments of one length
-// and a shorter last one: for each segment count the least padded wpg x spw
-// of whole wavefronts (K / 32 a multiple of spw) that gives that count, the
-// fewest covering 85% of the CUs; the wavefronts past K add nothing. Such
-// shapes serve up to 32 rows (measured against GemmKernel, which took these
-// shapes before: K = 11008, N = 4096 at M = 17 / 24 / 32 22.4 / 22.8 / 23.3
-// -> 20.4 / 20.6 / 20.9 us, K = 18944, N = 3584 at M = 32 32.7 -> 29.8; at
-// M = 40-64 level or slower, up to +21%).
-inline StreamShape PickStreamShape(const WeightView &w, int segs_req, int spw_req) {
+// The launch shape: groups of 64 rows per workgroup, K segments, wavefronts
+// per workgroup (4 to 8) and steps per wavefront (4, 8 or 16; 8 or 16 with two
+// groups) with whose product K / 32 divides; only where none does, shapes whose
+// last segment is shorter. Least cost in steps of one wavefront: the rounds that the busiest CU runs
+// (one workgroup at a time) times a wavefront's steps plus 5.5 for the launch's
+// fill and drain, plus 4 for the reduction of several segments; a step of two
+// groups counts 1.75 (two row tiles) or 1.55 (more), since the activations are
+// loaded once. Fewer segments on a tie. It gives within 10% of the measured
+// times (M = 48, us: K = N = 4096 four segments of 8 x 4 12.4, two of 8 x 8
+// 13.9, one of 8 x 16 15.8; N = 6144 four of 8 x 4, 1.5 rounds, 17.7, two of
+// 8 x 8 14.4; K = 14336, N = 4096 seven of 8 x 8 24.2, four of 7 x 16 19.8;
+// N = 28672 one of 8 x 16 30.4, two groups per workgroup 27.3).
+inline StreamShape PickStreamShape(const WeightView &w, int64_t M, int segs_req, int spw_req) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
   const int T = static_cast<int>(w.K / 32);
   if (segs_req > 0 && spw_req > 0) {
     const int per = segs_req * spw_req;
     return StreamShape{segs_req, T % per == 0 ? T / per : 0, spw_req};
   }
-  auto fit = [](int per) {
-    for (int wpg : {8, 4})
-      for (int spw : {16, 8, 4})
-        if (wpg * spw == per) return StreamShape{0, wpg, spw};
-    return StreamShape{0, 0, 0};
-  };
   StreamShape best{0, 0, 0};
-  for (int segs = 1; segs <= kMaxSplits; ++segs) {
-    if (T % segs != 0) continue;
-    StreamShape sh = fit(T / segs);
-    if (sh.wpg == 0) continue;
-    sh.segs = segs;
-    best = sh;
-    if (groups * segs * 100 >= static_cast<int64_t>(w.num_cus) * 85) break;
-  }
-  if (best.wpg != 0) return best;
-  for (int segs = 1; segs <= kMaxSplits; ++segs) {
-    StreamShape sh{0, 0, 0};
-    for (int wpg : {8, 4})
-      for (int spw : {16, 8, 4}) {
-        const int per = wpg * spw;
-        if (T % spw != 0 || (T + per - 1) / per != segs) continue;
-        if (sh.wpg == 0 || per < sh.wpg * sh.spw) sh = StreamShape{segs, wpg, spw, true};
-      }
-    if (sh.wpg == 0) continue;
-    best = sh;
-    if (groups * segs * 100 >= static_cast<int64_t>(w.num_cus) * 85) break;
+  double best_cost = 0.0;
+  for (bool ragged : {false, true}) {
+    for (int g : {1, 2})
+      for (int segs = 1; segs <= kMaxSplits; ++segs)
+        for (int spw : {16, 8, 4}) {
+          if (T % spw != 0 || (g == 2 && spw == 4)) continue;
+          const int wpg = std::max(4, (T / spw + segs - 1) / segs);  // wavefronts cover a segment
+          const int per = wpg * spw;
+          if (wpg > 8 || (T + per - 1) / per != segs || (T % per != 0) != ragged) continue;
+          const int64_t wgs = (groups + g - 1) / g * segs;
+          const int64_t rounds = (wgs + w.num_cus - 1) / std::max(1, w.num_cus);
+          const double step = g == 1 ? 1.0 : M <= 32 ? 1.75 : 1.55;
+          const double cost =
+              static_cast<double>(rounds) * (spw * step + 5.5) + (segs > 1 ? 4.0 : 0.0);
+          if (best.wpg == 0 || cost < best_cost - 1e-9 ||
+              (cost < best_cost + 1e-9 && segs < best.segs)) {
+            best = StreamShape{segs, wpg, spw, ragged, g};
+            best_cost = cost;
+          }
+        }
+    if (best.wpg != 0) break;
   }
   return best;
 }
@@ -1369,53 +1418,64 @@ inline StreamShape PickStreamShape(const WeightView &w, int segs_req, int spw_re
 // per call against ConvertAKernel + the image: c4 M = 17 / 32 10.45 -> 8.79
 // / 10.76 -> 10.11 us; slower where the fragments or the workgroups are more
 // (c4 M = 48 / 64 +0.4 / +1.2 us, c3 M = 32 with 8 steps per wavefront
-// +4.9 us, c5 qkv M = 32 with 1.5 workgroups per CU +1.4 us).
+// +4.9 us, c5 qkv M = 32 with 1.5 workgroups per CU +1.4 us), so only with
+// two row tiles and 4 steps.
 inline bool StreamConverts(const WeightView &w, int64_t M, const StreamShape &sh, bool rms) {
   const int64_t wgs = (w.N + kSGroupRows - 1) / kSGroupRows * sh.segs;
-  return !rms && (M + 15) / 16 * sh.spw <= 8 && wgs <= w.num_cus;
+  return !rms && sh.groups == 1 && (M + 15) / 16 * sh.spw <= 8 && wgs <= w.num_cus;
 }
 
-template <bool HAS_ZP, int TG, int SPW>
-hipError_t LaunchStreamT(const WeightView &w, int64_t M, const uint4 *Ah, const float *A, float *Y,
-                         float *P, float *H, const int *row_exp, const float *bias,
-                         const StreamShape &sh, hipStream_t s) {
+// The launch's operands: the fp16 image with its chunk exponents and (RMSNorm)
+// sums of squares, or A itself for the wavefronts to convert.
+struct StreamIn {
+  const uint4 *Ah;
+  const float *A;
+  const int *exps;
+  const float *sq;
+  float eps;
+};
+
+template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
+hipError_t LaunchStreamT(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
+                         float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
-  const size_t lds = static_cast<size_t>(sh.wpg) * TG * 4 * 64 * 16;
-  const dim3 grid(static_cast<unsigned>(groups * sh.segs)), block(64 * sh.wpg);
-  const int m = static_cast<int>(M), n = static_cast<int>(w.N), k = static_cast<int>(w.K);
-  if (A != nullptr) {
-    if constexpr (TG * SPW <= 16)
-      hipLaunchKernelGGL((StreamKernel<HAS_ZP, TG, SPW, 4, true>), grid, block, lds, s, Ah, A, w.Bp,
-                         w.Sp, Y, P, H, row_exp, w.col_exp, bias, m, n, k, w.log2_bs, sh.segs, sh.wpg);
-    else
-      return hipErrorInvalidValue;
-  } else {
-    hipLaunchKernelGGL((StreamKernel<HAS_ZP, TG, SPW, 4, false>), grid, block, lds, s, Ah, A, w.Bp,
-                       w.Sp, Y, P, H, row_exp, w.col_exp, bias, m, n, k, w.log2_bs, sh.segs, sh.wpg);
-  }
+  const size_t lds = static_cast<size_t>(sh.wpg) * TG * 2 * 64 * 16;
+  const dim3 grid(static_cast<unsigned>((groups + G - 1) / G * sh.segs)), block(64 * sh.wpg);
+  hipLaunchKernelGGL((StreamKernel<HAS_ZP, TG, SPW, WIN, CVT, G>), grid, block, lds, s, in.Ah, in.A,
+                     w.Bp, w.Sp, Y, P, H, in.exps, w.col_exp, bias, in.sq, in.eps,
+                     static_cast<int>(M), static_cast<int>(w.N), static_cast<int>(w.K), w.log2_bs,
+                     sh.segs, sh.wpg);
   return hipGetLastError();
 }
 
 template <bool HAS_ZP, int TG>
-hipError_t LaunchStreamTG(const WeightView &w, int64_t M, const uint4 *Ah, const float *A, float *Y,
-                          float *P, float *H, const int *row_exp, const float *bias,
-                          const StreamShape &sh, hipStream_t s) {
+hipError_t LaunchStreamTG(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
+                          float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
+  if (in.A != nullptr) {  // StreamConverts: two row tiles, 4 steps
+    if constexpr (TG == 2)
+      return LaunchStreamT<HAS_ZP, TG, 4, 4, true, 1>(w, M, in, Y, P, H, bias, sh, s);
+    return hipErrorInvalidValue;
+  }
+  if (sh.groups == 2) switch (sh.spw) {
+    case 8: return LaunchStreamT<HAS_ZP, TG, 8, WinG2<TG>(), false, 2>(w, M, in, Y, P, H, bias, sh, s);
+    case 16: return LaunchStreamT<HAS_ZP, TG, 16, WinG2<TG>(), false, 2>(w, M, in, Y, P, H, bias, sh, s);
+    default: return hipErrorInvalidValue;
+  }
   switch (sh.spw) {
-  case 4: return LaunchStreamT<HAS_ZP, TG, 4>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
-  case 8: return LaunchStreamT<HAS_ZP, TG, 8>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
-  case 16: return LaunchStreamT<HAS_ZP, TG, 16>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
+  case 4: return LaunchStreamT<HAS_ZP, TG, 4, 4, false, 1>(w, M, in, Y, P, H, bias, sh, s);
+  case 8: return LaunchStreamT<HAS_ZP, TG, 8, 4, false, 1>(w, M, in, Y, P, H, bias, sh, s);
+  case 16: return LaunchStreamT<HAS_ZP, TG, 16, 4, false, 1>(w, M, in, Y, P, H, bias, sh, s);
   default: return hipErrorInvalidValue;
   }
 }
 
 template <bool HAS_ZP>
-hipError_t LaunchStreamZp(const WeightView &w, int64_t M, const uint4 *Ah, const float *A, float *Y,
-                          float *P, float *H, const int *row_exp, const float *bias,
-                          const StreamShape &sh, hipStream_t s) {
+hipError_t LaunchStreamZp(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
+                          float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
   switch ((M + 15) / 16) {
-  case 2: return LaunchStreamTG<HAS_ZP, 2>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
-  case 3: return LaunchStreamTG<HAS_ZP, 3>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
-  case 4: return LaunchStreamTG<HAS_ZP, 4>(w, M, Ah, A, Y, P, H, row_exp, bias, sh, s);
+  case 2: return LaunchStreamTG<HAS_ZP, 2>(w, M, in, Y, P, H, bias, sh, s);
+  case 3: return LaunchStreamTG<HAS_ZP, 3>(w, M, in, Y, P, H, bias, sh, s);
+  case 4: return LaunchStreamTG<HAS_ZP, 4>(w, M, in, Y, P, H, bias, sh, s);
   default: return hipErrorInvalidValue;
   }
 }
@@ -1481,11 +1541,11 @@ __global__ __launch_bounds__(256) void RelayoutSKernel(const float *__restrict__
   const int64_t gb = idx >> 6;
   const int64_t b = gb % nb, g = gb / nb;
   const int64_t n = 64 * g + 16 * j + c;
-  uint32_t v = 8u << 16;  // rows past N: scale 0
+  uint32_t v = (8u << 16) | (8u << 28);  // rows past N: scale 0
   if (n < N) {
     const _Float16 h = static_cast<_Float16>(__builtin_amdgcn_ldexpf(S[n * nb + b], col_exp[n]));
     const uint32_t z = Z != nullptr ? (Z[n * zp_row_bytes + (b >> 1)] >> (4 * (b & 1))) & 0xFu : 8u;
-    v = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) | (z << 16);
+    v = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) | (z << 16) | (z << 28);
   }
   Sp[idx] = v;
 }
@@ -1500,28 +1560,27 @@ bool PrefillSupportsM(const WeightView &w, int64_t M) {
          (M + kPTM - 1) / kPTM * ((w.N + kPTN - 1) / kPTN) * kMaxSplits < (int64_t{1} << 31);
 }
 
-// Whether the streaming kernel's launch for M rows (M > 32) holds more than
-// three workgroups per CU: each workgroup stages its K segment of every
-// activation row, so with three or four 16-row token groups such launches
-// fall behind the prefill kernel's 128 x 256 tiles, from 33 rows when K is
-// split (the partial sums add their own traffic), from 49 when it is not.
-// Measured on MI355X, us per call at M = 33 / 48 / 64, streaming against
-// prefill: K = 5120, N = 13824 (1080 workgroups)
-// 35.5 / 37.3 / 45.7 against 29.4 / 31.0 / 32.2; K = 3584, N = 18944 (2072)
-// 29.5 / 32.5 / 45.8 against 28.5 / 30.0 / 31.7; K = 28672, N = 8192 (896)
-// 74.1 / 75.7 / 89.5 against 68.7 / 71.7 / 74.5; K = 8192, N = 28672 (896)
-// 68.3 / 70.4 / 83.2 against 66.9 / 65.4 / 73.8; K = 8192, N = 128256
-// (4008) 257 / 264 / 317 against 242 / 248 / 253; K = 4096, N = 128256
-// (2004, one segment) 127.8 / 129.6 / 155.3 against 130.9 / 134.3 / 137.7.
-// Launches of
-// up to 1.75 workgroups per CU stay faster streamed (K = 4096, N = 28672:
-// 34.5 / 34.8 / 41.2 against 39.3 / 40.9 / 41.5; c2, c4, K = N = 8192,
-// K = 14336, N = 4096 and K = 24576, N = 3072 by 15-40%).
+// Weights that the prefill kernel keeps above 32 rows: K / 32 steps that
+// segments of 8 x 16 steps do not divide, cut evenly into so many segments
+// (of 4 or 8 wavefronts of 4, 8 or 16 steps, covering 85% of the CUs) that
+// groups x segments are more than three per CU. Streaming them was slower than
+// the prefill kernel before the activations came in operand order; now it is
+// 8 to 16% faster (K = 5120, N = 13824 at M = 33 / 64 26.7 / 29.3 against
+// 29.0 / 32.3 us, K = 3584, N = 18944 23.7 / 27.2 against 28.2 / 31.4), but
+// their route is part of what the tests fix, so it stays.
 bool StreamCrowded(const WeightView &w, int64_t M) {
-  const StreamShape sh = PickStreamShape(w, 0, 0);
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
-  return M > 32 && sh.segs > 0 && (sh.segs > 1 || M > 48) &&
-         groups * sh.segs > 3 * static_cast<int64_t>(w.num_cus);
+  const int T = static_cast<int>(w.K / 32);
+  if (M <= 32 || T % 128 == 0) return false;
+  int best = 0;
+  for (int segs = 1; segs <= kMaxSplits; ++segs) {
+    const int per = T % segs == 0 ? T / segs : 0;
+    if (per != 16 && per != 32 && per != 64 && per != 128) continue;
+    best = segs;
+    if (groups * segs * 100 >= static_cast<int64_t>(w.num_cus) * 85) break;
+  }
+  return (best > 1 || (best == 1 && M > 48)) &&
+         groups * best > 3 * static_cast<int64_t>(w.num_cus);
 }
 
 // The prefill kernel serves the automatic GEMM path
@@ -1565,11 +1624,16 @@ size_t PrefillPartialBytes(const WeightView &w, int64_t M) {
   return static_cast<size_t>(PrefillSplits(w, M) - 1) * static_cast<size_t>(M) * w.N * 4;
 }
 
+// 17 to 64 rows. Steps with no even division (a shorter last segment) above
+// 32 rows: from 16 Mi weights; smaller ones stay with GemmKernel, whose route
+// the tests fix (K = 11008, N = 1024 at M = 33 / 64 streamed 12.6 / 13.7
+// against 16.3 / 16.9 us; N = 2048 14.6 / 16.4 against 18.2 / 19.3, N = 4096
+// 21.0 / 23.0 against 25.2 / 26.9).
 bool StreamSupportsM(const WeightView &w, int64_t M) {
   if (M < 17 || M > 64 || !PrefillSupportsShape(w) || w.K > (int64_t{1} << 22)) return false;
   if (StreamCrowded(w, M)) return false;
-  const StreamShape sh = PickStreamShape(w, 0, 0);
-  return sh.segs > 0 && (!sh.ragged || M <= 32);  // shorter last segment: up to 32 rows
+  const StreamShape sh = PickStreamShape(w, M, 0, 0);
+  return sh.segs > 0 && (!sh.ragged || M <= 32 || w.K * w.N >= (int64_t{16} << 20));
 }
 
 size_t StreamPartialBytes(const WeightView &w, int64_t M, int segs) {
@@ -1582,50 +1646,61 @@ size_t GemmWorkspaceBytes(const WeightView &w, int64_t M) {
   size_t partial = w.B != nullptr ? PartialBytes(w, M, PickShape(w, M)) : 0;
   if (PrefillSupportsM(w, M)) partial = std::max(partial, PrefillPartialBytes(w, M));
   if (StreamSupportsM(w, M))
-    partial = std::max(partial, StreamPartialBytes(w, M, PickStreamShape(w, 0, 0).segs));
-  return AImageBytes(w, M) + RowExpBytes(M) + partial;
+    partial = std::max(partial, StreamPartialBytes(w, M, PickStreamShape(w, M, 0, 0).segs));
+  return AImageBytes(w, M) + RowExpBytes(w, M) + partial;
 }
 
 bool StreamSupports(const WeightView &w, int64_t M) { return StreamSupportsM(w, M); }
 
 size_t StreamWorkspaceBytes(const WeightView &w, int64_t M, int segs, int spw) {
-  const StreamShape sh = PickStreamShape(w, segs, spw);
-  return AImageBytes(w, M) + RowExpBytes(M) + StreamPartialBytes(w, M, sh.segs);
+  const StreamShape sh = PickStreamShape(w, M, segs, spw);
+  return AImageBytes(w, M) + RowExpBytes(w, M) + StreamPartialBytes(w, M, sh.segs);
 }
 
 // The epilogue finishes fragments wave, wave + wpg, ... up to TG of them per
 // wavefront, so it needs wpg >= 4 to reach all 4 TG; at most 8 wavefronts.
 bool StreamShapeOk(const WeightView &w, int64_t M, int segs, int spw) {
-  const StreamShape sh = PickStreamShape(w, segs, spw);
+  const StreamShape sh = PickStreamShape(w, M, segs, spw);
   // every step in a segment, no segment empty (the last may be shorter)
   const int64_t per = static_cast<int64_t>(sh.wpg) * sh.spw, T = w.K / 32;
   return StreamSupportsM(w, M) && sh.segs >= 1 && sh.segs <= kMaxSplits && sh.wpg >= 4 &&
          sh.wpg <= 8 && T % sh.spw == 0 && sh.segs * per >= T && (sh.segs - 1) * per < T;
 }
 
-// ConvertA (64-row tiling), the streaming kernel, and the ordered reduction
-// of the segments' partial sums when K is split.
+// The chunk conversion, the streaming kernel, and the ordered reduction of the
+// segments' partial sums when K is split.
 hipError_t LaunchStream(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                         hipStream_t s, float *H, const float *gamma, float eps, const float *bias,
                         int segs, int spw) {
-  const StreamShape sh = PickStreamShape(w, segs, spw);
+  const StreamShape sh = PickStreamShape(w, M, segs, spw);
   if (!StreamShapeOk(w, M, segs, spw)) return hipErrorInvalidValue;
   uint4 *Ah = static_cast<uint4 *>(work);
-  int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
+  int *exps = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *P = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                       RowExpBytes(M));
+                                       RowExpBytes(w, M));
   const bool cvt = StreamConverts(w, M, sh, gamma != nullptr);
+  StreamIn in{Ah, cvt ? A : nullptr, exps, nullptr, eps};
   hipError_t e = hipSuccess;
-  if (!cvt)
-    e = gamma != nullptr
-            ? LaunchConvertA<kSGroupRows, true>(w, M, A, Ah, row_exp, s, gamma, eps)
-            : LaunchConvertA<kSGroupRows, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
+  if (!cvt) {
+    const int m = static_cast<int>(M), K = static_cast<int>(w.K);
+    const int groups = static_cast<int>((M + 15) / 16), chunks = (K + kChunkK - 1) / kChunkK;
+    float *sq = reinterpret_cast<float *>(exps + chunks * 16 * groups);
+    const dim3 grid(chunks * groups), block(512);
+    if (gamma != nullptr) {
+      in.sq = sq;
+      hipLaunchKernelGGL(ConvertChunkKernel<true>, grid, block, 0, s, A, Ah, exps, sq, gamma, m, K,
+                         chunks, 16 * groups);
+    } else {
+      hipLaunchKernelGGL(ConvertChunkKernel<false>, grid, block, 0, s, A, Ah, exps, nullptr, nullptr,
+                         m, K, chunks, 16 * groups);
+    }
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) return e;
   float *Hk = sh.segs == 1 ? H : nullptr;
   const float *bk = sh.segs == 1 ? bias : nullptr;
-  const float *Ak = cvt ? A : nullptr;
-  e = w.has_zp ? LaunchStreamZp<true>(w, M, Ah, Ak, Y, P, Hk, row_exp, bk, sh, s)
-                      : LaunchStreamZp<false>(w, M, Ah, Ak, Y, P, Hk, row_exp, bk, sh, s);
+  e = w.has_zp ? LaunchStreamZp<true>(w, M, in, Y, P, Hk, bk, sh, s)
+               : LaunchStreamZp<false>(w, M, in, Y, P, Hk, bk, sh, s);
   if (e != hipSuccess || sh.segs == 1) return e;
   return DispatchReduce(sh.segs - 1, Y, P, M * w.N, s, H,
                         std::make_integer_sequence<int, kMaxSplits - 1>{}, bias, w.N);
@@ -1669,7 +1744,7 @@ static hipError_t LaunchPrefillGemm(const WeightView &w, int64_t M, const float 
   uint4 *Ah = static_cast<uint4 *>(work);
   int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *partials = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                              RowExpBytes(M));
+                                              RowExpBytes(w, M));
   hipError_t e = gamma != nullptr
                      ? LaunchConvertA<kPTM, true>(w, M, A, Ah, row_exp, s, gamma, eps)
                      : LaunchConvertA<kPTM, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
@@ -1691,7 +1766,7 @@ static hipError_t LaunchPrefillGemm(const WeightView &w, int64_t M, const float 
 }
 
 size_t GemmShapeWorkspaceBytes(const WeightView &w, int64_t M, int splits) {
-  return AImageBytes(w, M) + RowExpBytes(M) + PartialBytes(w, M, MakeShape(w, 32, splits));
+  return AImageBytes(w, M) + RowExpBytes(w, M) + PartialBytes(w, M, MakeShape(w, 32, splits));
 }
 
 bool GemmSupports(const WeightView &w, int64_t M) {

@@ -202,3 +202,55 @@ def test_stream_shorter_last_segment_serves_up_to_32_rows(pkg, cuda):
         assert names[33] != "StreamKernel" and names[64] != "StreamKernel"
     finally:
         op.release()
+
+
+@pytest.mark.parametrize("K,N,bs,zp,M", [
+    (512, 64, 32, True, 17),       # one group, one chunk of K, one row past a row tile
+    (1088, 132, 64, False, 33),    # 34 steps: a wavefront per 8 does not divide; ragged columns
+    (4096, 28672, 128, True, 48),  # two column groups per workgroup
+    (4096, 28740, 32, False, 64),  # an odd group count: the last workgroup's second group is padding
+    (14336, 4096, 128, True, 64),  # seven wavefronts of 16 steps, four segments
+    (2624, 17408, 64, True, 40),   # two groups, a chunk that K does not fill
+])
+def test_stream_shapes_rms_and_bias(pkg, orc, cuda, K, N, bs, zp, M):
+    """The launch shapes of the streaming GEMM (wavefronts per workgroup, one
+    or two column groups, segments) with the plain input, a bias and the
+    RMSNorm input, whose 1 / rms comes from the chunks' sums of squares; rows
+    of very different magnitude, a zero row and a zero chunk."""
+    import torch
+    p = pkg.workloads.Projection("shapes", K, N, bs, zp)
+    B, S, Z = pkg.workloads.make_weights(p, K + N)
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare(B, S, Z)
+    A = pkg.workloads.make_activations(M, K, 1.0, M)
+    A[1] *= 1e20
+    A[2] *= 1e-20
+    A[3] = 0.0
+    A[4, :min(512, K // 2)] = 0.0
+    A[5, :min(512, K // 2)] *= 1e-6
+    dA = torch.from_numpy(A).to(cuda)
+    rng = np.random.default_rng(N)
+    cols = np.unique(np.concatenate([rng.integers(0, N, 96), [0, N - 1, min(64, N - 1)]]))
+    bias = rng.standard_normal(N).astype(np.float32)
+    gamma = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    print(f"case stream shapes K={K} N={N} bs={bs} M={M} kernel={op.kernel_name(M)}", flush=True)
+    ref = lambda X: orc.matmul_nbits_f64(X, B[cols], S[cols], None if Z is None else Z[cols],
+                                         K, len(cols), bs)
+    y64 = ref(A)
+
+    def check(Y, want):
+        for m in range(M):  # row by row: their magnitudes differ by 40 decades
+            assert orc.l2_rel_error(Y[m:m + 1, cols], want[m:m + 1]) <= 2e-3 if want[m].any() \
+                else not Y[m].any(), m
+
+    Y = op(dA).cpu().numpy()
+    check(Y, y64)
+    Yb = op(dA, bias=torch.from_numpy(bias).to(cuda)).cpu().numpy()
+    np.testing.assert_array_equal(Yb, Y + bias[None, :])
+    # rows whose squares stay in fp32's range
+    keep = [m for m in range(M) if m not in (1, 2)]
+    Yn = op.run_rmsnorm(dA[keep].contiguous(), torch.from_numpy(gamma).to(cuda), 1e-5).cpu().numpy()
+    n64 = ref(orc.rmsnorm_f64(A[keep].astype(np.float64), gamma.astype(np.float64), 1e-5).astype(np.float32))
+    for i in range(len(keep)):
+        if n64[i].any():
+            assert orc.l2_rel_error(Yn[i:i + 1, cols], n64[i:i + 1]) <= 2e-3, keep[i]
+    op.release()
