@@ -1119,6 +1119,7 @@ const char *mnb_kernel_name(const mnb_plan *plan, int64_t M, size_t workspace_by
     }
   case 2:
     return mnb::GemmUsesStream(plan->view, M)    ? "StreamKernel"
+           : mnb::GemmUsesWide(plan->view, M)    ? "WideKernel"
            : mnb::GemmUsesPrefill(plan->view, M) ? "PrefillKernel"
                                                  : "GemmKernel";
   case 4: return "exact groups of 16 rows";

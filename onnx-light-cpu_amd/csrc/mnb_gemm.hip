@@ -1620,6 +1620,33 @@ bool UsePrefill(const WeightView &w, int64_t M) {
   return last * 2 >= cus;
 }
 
+// The wide kernel, by waves of one workgroup per CU: one of its tiles takes
+// 1.75 times a PrefillKernel tile (about 112 and 64 us at K = 4096) for twice
+// the work, so it wins unless its last wave is emptier than the prefill
+// kernel's by more than that (M = 700, N = 28672: 2 waves against 3, 208
+// against 189 us). Where GemmKernel would serve, whose time goes with the
+// work, 1.33 prefill waves per full wave of 128 x 256 tiles. Fewer tiles than
+// CUs are the prefill kernel's (it splits K). Measured (us, prefill or
+// GemmKernel -> wide): K = 4096, N = 28672 at M = 448 / 512 / 1024 / 1280 /
+// 1536 / 2048 / 8192 128.8 -> 113.4, 132.8 -> 114.9, 262 -> 226, 369 -> 325,
+// 445 -> 329, 448 -> 434, 1877 -> 1675 (with streaming stores, 1 to 6% slower
+// than the plain ones that it has); N = 6144 at M = 2048 / 2560 / 8192
+// 130 -> 112, 137 -> 127, 422 -> 376; K = 14336, N = 4096 at M = 3584 / 8192
+// 431 -> 388, 928 -> 858; K = 8192, N = 8192 at M = 2048 257 -> 235. Below
+// K = 2048 the un-overlapped prologue and stores of the larger tile take it
+// back (K = 1024, N = 8192, M = 2048: 56.1 -> 57.8).
+bool UseWide(const WeightView &w, int64_t M) {
+  // 32-bit offsets within a tile's rows.
+  if (!PrefillSupportsM(w, M) || w.K < 2048 || w.N >= (int64_t{1} << 21)) return false;
+  const int64_t cus = w.num_cus;
+  const int64_t tiles = (M + kPTM - 1) / kPTM * ((w.N + kPTN - 1) / kPTN);
+  if (tiles < cus) return false;
+  const int64_t wide = (M + kWideRows - 1) / kWideRows * ((w.N + kWideCols - 1) / kWideCols);
+  const int64_t cost = 7 * ((wide + cus - 1) / cus) * cus;  // a prefill wave: 4 cus
+  return UsePrefill(w, M) || w.B == nullptr ? cost <= 4 * ((tiles + cus - 1) / cus) * cus
+                                            : cost * 3 <= 16 * tiles;
+}
+
 size_t PrefillPartialBytes(const WeightView &w, int64_t M) {
   return static_cast<size_t>(PrefillSplits(w, M) - 1) * static_cast<size_t>(M) * w.N * 4;
 }
@@ -1765,6 +1792,20 @@ static hipError_t LaunchPrefillGemm(const WeightView &w, int64_t M, const float 
                         std::make_integer_sequence<int, kMaxSplits - 1>{}, bias, w.N);
 }
 
+// ConvertA and the wide kernel, which applies the gate/up activation or adds
+// the bias in its stores.
+static hipError_t LaunchWideGemm(const WeightView &w, int64_t M, const float *A, float *Y,
+                                 void *work, hipStream_t s, float *H, const float *gamma,
+                                 float eps, const float *bias) {
+  uint4 *Ah = static_cast<uint4 *>(work);
+  int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
+  const hipError_t e = gamma != nullptr
+                           ? LaunchConvertA<16, true>(w, M, A, Ah, row_exp, s, gamma, eps)
+                           : LaunchConvertA<16, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
+  if (e != hipSuccess) return e;
+  return LaunchWide(w, M, Ah, Y, H, row_exp, bias, s);
+}
+
 size_t GemmShapeWorkspaceBytes(const WeightView &w, int64_t M, int splits) {
   return AImageBytes(w, M) + RowExpBytes(w, M) + PartialBytes(w, M, MakeShape(w, 32, splits));
 }
@@ -1821,7 +1862,12 @@ hipError_t LaunchGemm(const WeightView &w, int64_t M, const float *A, float *Y, 
     if (bias_done != nullptr) *bias_done = bias != nullptr;
     return LaunchStream(w, M, A, Y, work, s, H, gamma, eps, bias, 0, 0);
   }
-  // A compact plan (no original layout) always takes the prefill kernel.
+  if (UseWide(w, M)) {
+    if (bias_done != nullptr) *bias_done = bias != nullptr;
+    return LaunchWideGemm(w, M, A, Y, work, s, H, gamma, eps, bias);
+  }
+  // A compact plan (no original layout) always takes one of the kernels on the
+  // re-laid weights.
   if (UsePrefill(w, M) || w.B == nullptr) {
     if (bias_done != nullptr) *bias_done = bias != nullptr;
     return LaunchPrefillGemm(w, M, A, Y, work, s, H, gamma, eps, bias, PrefillSplits(w, M));
@@ -1832,5 +1878,9 @@ hipError_t LaunchGemm(const WeightView &w, int64_t M, const float *A, float *Y, 
 bool GemmUsesPrefill(const WeightView &w, int64_t M) { return UsePrefill(w, M) || w.B == nullptr; }
 
 bool GemmUsesStream(const WeightView &w, int64_t M) { return StreamSupportsM(w, M); }
+
+bool GemmUsesWide(const WeightView &w, int64_t M) {
+  return !StreamSupportsM(w, M) && UseWide(w, M);
+}
 
 } // namespace mnb

@@ -246,15 +246,17 @@ hipError_t LaunchSumPartials(float *Y, const float *P, int64_t mn, int parts, fl
 // holds GemmWorkspaceBytes(w, M) bytes of device memory: A scaled per row by
 // a power of two and rounded to fp16, the rows' exponents, then the partial
 // sums of a split-K launch.
-// On a plan holding the re-laid weights, StreamKernel serves 17 <= M <= 64
-// and the prefill kernel (128 x 256 tiles) M >= 65 where its tiles fill the
-// CUs; both add `bias` (N floats) themselves and then set *bias_done.
+// On a plan holding the re-laid weights, StreamKernel serves 17 <= M <= 64,
+// WideKernel (256 x 256 tiles) and the prefill kernel (128 x 256 tiles) M >= 65
+// where their tiles fill the CUs; all three add `bias` (N floats) themselves
+// and then set *bias_done.
 // Otherwise GemmKernel (BM x 128 tiles over the original layout) serves.
 hipError_t LaunchGemm(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                       hipStream_t s, float *H = nullptr, const float *gamma = nullptr,
                       float eps = 0.0f, const float *bias = nullptr, bool *bias_done = nullptr);
 bool GemmUsesPrefill(const WeightView &w, int64_t M);
 bool GemmUsesStream(const WeightView &w, int64_t M);
+bool GemmUsesWide(const WeightView &w, int64_t M);
 // The prefill kernel forced (any M >= 1 on a plan holding the re-laid
 // weights; split-K when its tiles alone do not fill the CUs); adds `bias`
 // in its epilogue and sets *bias_done.
@@ -276,6 +278,12 @@ bool StreamShapeOk(const WeightView &w, int64_t M, int segs, int spw);
 hipError_t LaunchStream(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                         hipStream_t s, float *H, const float *gamma, float eps, const float *bias,
                         int segs, int spw);
+// WideKernel (mnb_wide.hip) over the 16-row fp16 image of ConvertA: one
+// workgroup per tile of kWideRows x kWideCols. Adds `bias` itself (not with H).
+constexpr int kWideRows = 256;
+constexpr int kWideCols = 256;
+hipError_t LaunchWide(const WeightView &w, int64_t M, const uint4 *Ah, float *Y, float *H,
+                      const int *row_exp, const float *bias, hipStream_t s);
 // The prefill kernel's weight layout: whether the plan's shape can use it,
 // its byte sizes (Bp returned, Sp through sp_bytes), and the plan-time
 // re-layout from B, scales, zero points and col_exp.
