@@ -9,7 +9,8 @@
 // activation keeps 22 significant bits (relative error at most 2^-22, against
 // fp32's 2^-24 rounding of each product) and the products are summed in fp32.
 //
-// Two kernels per call:
+// Two kernels per call (one on small weights, where DecodeFragKernel does the
+// split itself: SplitInKernel):
 //
 // 1. SplitActKernel (one wavefront per unit of 256 k and pair of tokens)
 //    scales each token's values in the unit by a power of two 2^e (largest
@@ -34,8 +35,8 @@
 //    6.1 us against 7.9-8.6 us for 64-byte pieces of 16 rows). A third
 //    activation term (exact products) cost 15-25% more time on c1-c3 at
 //    M = 16 for no gain under the decode bound.
-//    - A workgroup of WPG wavefronts owns one group and a run of
-//      WPG * U consecutive units; wavefront w multiplies U of them. Per step
+//    - A workgroup of WPG wavefronts owns one group (or two, which share the
+//      operands: GroupPairs) and a run of WPG * U consecutive units; wavefront w multiplies U of them. Per step
 //      it decodes the record's four words (q - zp exact in fp16, exponent
 //      constants), reads the two activation terms of the step (from L2:
 //      the image is shared by every group) and issues 2 x 4
@@ -155,45 +156,56 @@ __global__ __launch_bounds__(64) void SplitActKernel(const float *__restrict__ A
   }
 }
 
-// Group g of 64 weight rows, run `seg` of WPG * U units. SPB = 32-k steps
+// G groups of 64 weight rows, run `seg` of WPG * U units. SPB = 32-k steps
 // per quantization block within a unit (bs / 32, at most 8).
 // RMS: the image holds A * gamma; every run scales its sums by each token's
 // 1 / rms = 1 / sqrt(sum_k A^2 / K + eps), from SplitActKernel's per-unit
 // sums of squares added in unit order.
-template <bool HAS_ZP, int SPB, int U, int WIN, bool RMS, int TOKS>
+// SPLIT (not RMS): img and exps are not read; the wavefront loads its units'
+// fp32 activations (the same bytes) a unit ahead and forms SplitActKernel's
+// terms and exponents from them, bit for bit.
+template <bool HAS_ZP, int SPB, int U, int WIN, bool RMS, int TOKS, int G, bool SPLIT>
 __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
     const uint8_t *__restrict__ Bp, const float *__restrict__ Sd, const uint32_t *__restrict__ Zd,
-    const uint4 *__restrict__ img, const int *__restrict__ exps, float *__restrict__ Y,
-    float *__restrict__ partials, float *__restrict__ H, const float *__restrict__ bias, int M,
+    const uint4 *__restrict__ img, const int *__restrict__ exps, const float *__restrict__ A,
+    float *__restrict__ Y, float *__restrict__ partials, float *__restrict__ H, const float *__restrict__ bias, int M,
     int N, int K, int nb, int log2_bs, int segs, int wpg, const float *__restrict__ sq,
     float eps) {
-  __shared__ float red[kMaxWaves * 16 * 64];  // 32 KiB: [wave][slice * 4 + v][lane]
+  __shared__ float red[kMaxWaves * 16 * G * 64];  // [wave][group, slice, v][lane]
   __shared__ float rinv[kTok];                // RMS: each token's 1 / rms
   __shared__ float sqs[RMS ? kMaxSqUnits * kTok : 1];  // RMS: the per-unit sums of squares
   constexpr int kSteps = U * kUnitSteps;
   constexpr int kSB = StepBytesT<TOKS>();
   constexpr int kTPL = TOKS / 4;     // tokens per lane in the MFMA result
-  constexpr int kItems = 4 * kTPL;   // (slice, token) results per lane
+  constexpr int kItems = 4 * kTPL * G;  // (group, slice, token) results per lane
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int c = lane & 15, qd = lane >> 4;
-  const int g = static_cast<int>(blockIdx.x) / segs;
-  const int seg = static_cast<int>(blockIdx.x) - g * segs;
+  const int gp = static_cast<int>(blockIdx.x) / segs;
+  const int seg = static_cast<int>(blockIdx.x) - gp * segs;
+  const int groups = (N + 63) / 64;
   const int T = K / 32;
   const int Tp = (K + kUnitK - 1) / kUnitK * kUnitSteps;  // steps of whole units (image, exponents)
   const int u0 = (seg * wpg + wave) * U;  // first unit of this wavefront
   const int s0 = u0 * kUnitSteps;         // first step
 
   // Per-group bases (wave-uniform), per-lane offsets below 2^31.
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t *>(Bp + static_cast<size_t>(g) * T * 1024), 0, T * 1024, 0x00020000);
   const __amdgpu_buffer_rsrc_t ri =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4 *>(img), 0, Tp * kSB, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(Sd + static_cast<size_t>(g) * nb * 64), 0, nb * 256, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint32_t *>(HAS_ZP ? Zd + static_cast<size_t>(g) * nb * 16 : Zd), 0,
-      HAS_ZP ? nb * 64 : 0, 0x00020000);
+  // A group past the last (an odd count) reads nothing but zeros.
+  __amdgpu_buffer_rsrc_t rb[G], rs[G], rz[G];
+#pragma unroll
+  for (int x = 0; x < G; ++x) {
+    const int g = min(gp * G + x, groups - 1);
+    const int on = gp * G + x < groups ? 1 : 0;
+    rb[x] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(Bp + static_cast<size_t>(g) * T * 1024), 0, on * T * 1024, 0x00020000);
+    rs[x] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(Sd + static_cast<size_t>(g) * nb * 64), 0, on * nb * 256, 0x00020000);
+    rz[x] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t *>(HAS_ZP ? Zd + static_cast<size_t>(g) * nb * 16 : Zd), 0,
+        HAS_ZP ? on * nb * 64 : 0, 0x00020000);
+  }
 
   // RMS: wavefront 0 copies the per-unit sums of squares ([unit][token],
   // 64 bytes per unit, L2-resident) straight into LDS first, with no
@@ -212,37 +224,67 @@ __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
   // Each unit's token exponents: lane quarter qd holds tokens kTPL qd ..
   // kTPL qd + kTPL - 1.
   int4 ue[U];
-  const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int *>(exps), 0, (Tp / kUnitSteps) * 64, 0x00020000);
+  if constexpr (!SPLIT) {
+    const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int *>(exps), 0, (Tp / kUnitSteps) * 64, 0x00020000);
 #pragma unroll
-  for (int uu = 0; uu < U; ++uu) {
-    if constexpr (TOKS == 16) {
-      ue[uu] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(re, (u0 + uu) * 64 + 16 * qd, 0, 0));
-    } else {
-      typedef int i32x2 __attribute__((ext_vector_type(2)));
-      const i32x2 e2 = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(re, (u0 + uu) * 64 + 8 * qd, 0, 0));
-      ue[uu] = int4{e2[0], e2[1], 0, 0};
+    for (int uu = 0; uu < U; ++uu) {
+      if constexpr (TOKS == 16) {
+        ue[uu] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(re, (u0 + uu) * 64 + 16 * qd, 0, 0));
+      } else {
+        typedef int i32x2 __attribute__((ext_vector_type(2)));
+        const i32x2 e2 = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(re, (u0 + uu) * 64 + 8 * qd, 0, 0));
+        ue[uu] = int4{e2[0], e2[1], 0, 0};
+      }
     }
   }
 
+  // SPLIT: the unit's fp32 activations of this lane's operand row, 8 values a
+  // step; tokens past M and steps past K read past the buffer's end: zeros.
+  const int a_end = M * K * 4;
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, SPLIT ? a_end : 0, 0x00020000);
+  const int a_tok = TOKS == 16 ? c : c >> 1;
+  const int a_off = (a_tok * K + 8 * qd) * 4;
+  floatx4 raw[SPLIT ? kUnitSteps : 1][2];
+  auto issueA = [&](int i) __attribute__((always_inline)) {
+    const int s = s0 + i;
+    const int vo = s < T && a_tok < M ? a_off + s * 128 : a_end;
+    raw[i % kUnitSteps][0] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra, vo, 0, 0));
+    raw[i % kUnitSteps][1] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra, vo + 16, 0, 0));
+  };
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < kUnitSteps; ++i) issueA(i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   struct Slot {
-    u32x4 w, a0, a1;
-    floatx4 s;
-    uint32_t z;
+    u32x4 w[G], a0, a1;
+    floatx4 s[G];
+    uint32_t z[G];
   };
   Slot ring[WIN];
   auto issue = [&](int i) __attribute__((always_inline)) {
     Slot &sl = ring[i % WIN];
     const int s = s0 + i;
-    sl.w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, s * 1024 + 16 * lane, 0,
-                                                                           kNonTemporal));
-    sl.a0 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ri, s * kSB + 16 * lane, 0, 0));
-    if constexpr (TOKS == 16)
+#pragma unroll
+    for (int x = 0; x < G; ++x)
+      sl.w[x] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              rb[x], s * 1024 + 16 * lane, 0, kNonTemporal));
+    if constexpr (!SPLIT)
+      sl.a0 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ri, s * kSB + 16 * lane, 0, 0));
+    if constexpr (!SPLIT && TOKS == 16)
       sl.a1 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ri, s * kSB + 1024 + 16 * lane, 0, 0));
     if (i % SPB == 0) {
       const int blk = (s * 32) >> log2_bs;
-      sl.s = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, blk * 256 + 16 * c, 0, 0));
-      if constexpr (HAS_ZP) sl.z = __builtin_amdgcn_raw_buffer_load_b32(rz, blk * 64 + 4 * c, 0, 0);
+#pragma unroll
+      for (int x = 0; x < G; ++x) {
+        sl.s[x] = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs[x], blk * 256 + 16 * c, 0, 0));
+        if constexpr (HAS_ZP)
+          sl.z[x] = __builtin_amdgcn_raw_buffer_load_b32(rz[x], blk * 64 + 4 * c, 0, 0);
+      }
     }
   };
 #pragma unroll
@@ -250,67 +292,111 @@ __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
   __builtin_amdgcn_sched_barrier(0);
 
   const Masks mk = MakeMasks();
-  floatx4 acc[4], racc[4], tmp[4];
-  floatx4 bsc = floatx4{0.f, 0.f, 0.f, 0.f};
-  uint32_t neg_lo[4], neg_hi[4];
+  // index 4 x + j: slice j of the workgroup's group x
+  floatx4 acc[4 * G], racc[4 * G], tmp[4 * G], bsc[G];
+  uint32_t neg_lo[4 * G], neg_hi[4 * G];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    neg_lo[j] = 0xE408E408u;  // fp16 -(1024 + 8)
-    neg_hi[j] = 0xD480D480u;  // fp16 -(64 + 8)
+  for (int y = 0; y < 4 * G; ++y) {
+    acc[y] = floatx4{0.f, 0.f, 0.f, 0.f};
+    neg_lo[y] = 0xE408E408u;  // fp16 -(1024 + 8)
+    neg_hi[y] = 0xD480D480u;  // fp16 -(64 + 8)
   }
+  int se = 0;  // SPLIT: the exponent of this lane's token in the current unit
   auto step = [&](int i) __attribute__((always_inline)) {
     Slot &sl = ring[i % WIN];
     // Pins the step's arithmetic here: left free, the compiler hoists work
     // on later steps' registers into this one and waits for their loads.
-    __asm__ volatile("" : "+v"(sl.w), "+v"(sl.a0), "+v"(sl.a1));
+#pragma unroll
+    for (int x = 0; x < G; ++x) __asm__ volatile("" : "+v"(sl.w[x]));
+    if constexpr (SPLIT) {
+      if (i % kUnitSteps == 0) {
+        // the unit's exponent per token, as SplitActKernel's
+        float amax = 0.f;
+#pragma unroll
+        for (int k = 0; k < kUnitSteps; ++k)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            amax = fmaxf(amax, fmaxf(fabsf(raw[k][0][v]), fabsf(raw[k][1][v])));
+        amax = fmaxf(amax, Xor16(amax));
+        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        se = RangeExponent(amax, 14);
+        int ev[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int v = 0; v < kTPL; ++v) ev[v] = __shfl(se, (16 / TOKS) * (kTPL * qd + v));
+        ue[i / kUnitSteps] = int4{ev[0], ev[1], ev[2], ev[3]};
+      }
+      half8 h0, h1;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        const int o = (v & 3) * 2 + (v >> 2);  // k order [0,4,1,5,2,6,3,7]
+        const float x = __builtin_amdgcn_ldexpf(raw[i % kUnitSteps][v >> 2][v & 3], se);
+        h0[o] = static_cast<_Float16>(x);
+        // exact; NaN where x is infinite or NaN, whose second term is 0
+        const float r = __builtin_fmaf(static_cast<float>(h0[o]), -1.0f, x);
+        h1[o] = static_cast<_Float16>(r == r ? r : 0.f);
+      }
+      sl.a0 = __builtin_bit_cast(u32x4, TOKS == 16 || (c & 1) == 0 ? h0 : h1);
+      sl.a1 = __builtin_bit_cast(u32x4, h1);
+      if (i + kUnitSteps < kSteps) issueA(i + kUnitSteps);
+    } else {
+      __asm__ volatile("" : "+v"(sl.a0), "+v"(sl.a1));
+    }
     if (i % kUnitSteps == 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) racc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int y = 0; y < 4 * G; ++y) racc[y] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
     if (i % SPB == 0) {
-      bsc = sl.s;
-      if constexpr (HAS_ZP) {
-        const uint32_t z = sl.z;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          // byte j is the zero point of row 16 j + c: fp16 -(1024 + zp) =
-          // 0xE400 | zp, -(64 + zp) = 0xD400 | zp << 4
-          const uint32_t zz = ((z >> (8 * j)) & 0xFu) * 0x10001u;
-          neg_lo[j] = zz | 0xE400E400u;
-          neg_hi[j] = (zz << 4) | 0xD400D400u;
+      for (int x = 0; x < G; ++x) {
+        bsc[x] = sl.s[x];
+        if constexpr (HAS_ZP) {
+          const uint32_t z = sl.z[x];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            // byte j is the zero point of row 16 j + c: fp16 -(1024 + zp) =
+            // 0xE400 | zp, -(64 + zp) = 0xD400 | zp << 4
+            const uint32_t zz = ((z >> (8 * j)) & 0xFu) * 0x10001u;
+            neg_lo[4 * x + j] = zz | 0xE400E400u;
+            neg_hi[4 * x + j] = (zz << 4) | 0xD400D400u;
+          }
         }
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) tmp[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int y = 0; y < 4 * G; ++y) tmp[y] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    half8 q[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = DecodeQ(sl.w[j], neg_lo[j], neg_hi[j], mk);
     const half8 a0 = __builtin_bit_cast(half8, sl.a0);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) tmp[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, q[j], tmp[j], 0, 0, 0);
-    if constexpr (TOKS == 16) {
-      const half8 a1 = __builtin_bit_cast(half8, sl.a1);
+    for (int x = 0; x < G; ++x) {
+      half8 q[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) tmp[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, q[j], tmp[j], 0, 0, 0);
+      for (int j = 0; j < 4; ++j)
+        q[j] = DecodeQ(sl.w[x][j], neg_lo[4 * x + j], neg_hi[4 * x + j], mk);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        tmp[4 * x + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, q[j], tmp[4 * x + j], 0, 0, 0);
+      if constexpr (TOKS == 16) {
+        const half8 a1 = __builtin_bit_cast(half8, sl.a1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          tmp[4 * x + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, q[j], tmp[4 * x + j], 0, 0, 0);
+      }
     }
     if ((i + 1) % SPB == 0) {
       // TOKS = 8: result rows 4 qd + v hold term v & 1 of token 2 qd + v / 2
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int y = 0; y < 4 * G; ++y)
 #pragma unroll
         for (int v = 0; v < kTPL; ++v)
-          racc[j][v] = fmaf(bsc[j], TOKS == 16 ? tmp[j][v] : tmp[j][2 * v] + tmp[j][2 * v + 1],
-                            racc[j][v]);
+          racc[y][v] = fmaf(bsc[y / 4][y % 4], TOKS == 16 ? tmp[y][v] : tmp[y][2 * v] + tmp[y][2 * v + 1],
+                            racc[y][v]);
     }
     if ((i + 1) % kUnitSteps == 0) {
       const int4 e4 = ue[i / kUnitSteps];
       const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int y = 0; y < 4 * G; ++y)
 #pragma unroll
-        for (int v = 0; v < kTPL; ++v) acc[j][v] += __builtin_amdgcn_ldexpf(racc[j][v], -ev[v]);
+        for (int v = 0; v < kTPL; ++v) acc[y][v] += __builtin_amdgcn_ldexpf(racc[y][v], -ev[v]);
     }
   };
   // Straight-line code (no loop, no branch around a load) keeps the
@@ -327,7 +413,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
   // The wavefronts' sums meet in LDS; wavefront w then finishes the (slice,
   // token) pairs x = w, w + wpg, ...: added in wavefront order.
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 4 * G; ++j)
 #pragma unroll
     for (int v = 0; v < kTPL; ++v) red[(wave * kItems + j * kTPL + v) * 64 + lane] = acc[j][v];
   if constexpr (RMS) {
@@ -351,7 +437,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
     float sum = red[x * 64 + lane];
     for (int w = 1; w < wpg; ++w) sum += red[(w * kItems + x) * 64 + lane];
     const int j = x / kTPL, v = x % kTPL;
-    const int n = 64 * g + 16 * j + c;
+    const int n = 64 * G * gp + 16 * j + c;
     const int tok = kTPL * qd + v;
     if constexpr (RMS) sum *= rinv[tok];
     if (H != nullptr) {
@@ -487,6 +573,36 @@ inline Shape PickShapeU12(const WeightView &w, int wpg_req, int u_req) {
   return sh;
 }
 
+// Above 8 tokens, two groups per workgroup: a step's 2 KiB of operands then
+// feed two records of weights instead of one. Those reads, not the weights',
+// are most of what a CU draws from its L2 (186 MB at K = 4096, N = 28672
+// against 62 MB of weights). Workgroups of 6 to 8 wavefronts, one per CU at a
+// time: a round of pairs takes 1.8 times a round of single groups, so pairs
+// are taken where they need 5/9 of the rounds or fewer. us at M = 16, single
+// -> pairs: K = 4096, N = 28672 (2 rounds, 1) 23.4 -> 21.4, N = 51200 (4, 2)
+// 40.5 -> 36.3, N = 128256 (8, 4) 82.7 -> 73.8; K = 14336, N = 16384 (2, 1)
+// 41.9 -> 35.5; not N = 33280 (3, 2) 30.1 -> 32.1, N = 14336 (1, 1) 14.4 ->
+// 17.9. Up to 8 tokens (1 KiB of operands a step) pairs are no faster (59.0 ->
+// 61.2 at N = 128256).
+inline bool GroupPairs(const WeightView &w, const Shape &sh) {
+  const int64_t groups = (w.N + 63) / 64, cus = std::max<int64_t>(1, w.num_cus);
+  const int64_t rounds = (groups * sh.segs + cus - 1) / cus;
+  const int64_t pair_rounds = ((groups + 1) / 2 * sh.segs + cus - 1) / cus;
+  return sh.wpg >= 6 && 9 * pair_rounds <= 5 * rounds;
+}
+
+// The main kernel splits the fp32 activations itself, without SplitActKernel's
+// launch, where every wavefront has one unit and there is at most one
+// wavefront per SIMD: the split then costs less than the launch. us at M = 5 /
+// 16: K = 4096, N = 4096 8.9 / 10.1 -> 7.9 / 9.4; K = 2048, N = 2048 8.9 /
+// 10.0 -> 7.6 / 9.0. With more wavefronts per SIMD each splits again what the
+// others did (K = 4096, N = 6144, 1.5 per SIMD, 10.2 / 11.8 -> 9.9 / 12.1;
+// K = 14336, N = 4096, two units each, 13.6 / 16.5 -> 14.6 / 18.0).
+inline bool SplitInKernel(const WeightView &w, const Shape &sh) {
+  return sh.units_per_wave == 1 &&
+         (w.N + 63) / 64 * sh.segs * sh.wpg <= 4 * std::max<int64_t>(1, w.num_cus);
+}
+
 inline size_t ImageBytes(const WeightView &w) {
   return static_cast<size_t>(Units(w)) * kUnitSteps * kStepBytes;
 }
@@ -502,27 +618,42 @@ struct Work {
   const uint4 *img;
   const int *exps;
   const float *sq;
+  const float *A;  // split in the kernel itself, else null
   float *P;
   float eps;
 };
 
-template <bool HAS_ZP, int SPB, int U, int TOKS>
-hipError_t LaunchMain(const WeightView &w, int64_t M, const Work &wk, float *Y, float *H,
+template <bool HAS_ZP, int SPB, int U, int TOKS, int G, bool SPLIT>
+hipError_t LaunchMainG(const WeightView &w, int64_t M, const Work &wk, float *Y, float *H,
                       const float *bias, const Shape &sh, hipStream_t s) {
   const int64_t groups = (w.N + 63) / 64;
-  constexpr int kWin = 4;
-  const dim3 grid(static_cast<unsigned>(groups * sh.segs)), block(64 * sh.wpg);
+  constexpr int kWin = 4;  // 6 and 8 steps: K = 4096, N = 128256 at M = 16 82.7 -> 84.0 / 87.0 us
+  const dim3 grid(static_cast<unsigned>((groups + G - 1) / G * sh.segs)), block(64 * sh.wpg);
   const int m = static_cast<int>(M), n = static_cast<int>(w.N), k = static_cast<int>(w.K),
             nb = static_cast<int>(w.nb);
   if (wk.sq != nullptr)
-    hipLaunchKernelGGL((DecodeFragKernel<HAS_ZP, SPB, U, kWin, true, TOKS>), grid, block, 0, s, w.Bp,
-                       w.Sd, w.Zd, wk.img, wk.exps, Y, wk.P, H, bias, m, n, k, nb, w.log2_bs,
+    hipLaunchKernelGGL((DecodeFragKernel<HAS_ZP, SPB, U, kWin, true, TOKS, G, false>), grid, block, 0, s, w.Bp,
+                       w.Sd, w.Zd, wk.img, wk.exps, wk.A, Y, wk.P, H, bias, m, n, k, nb, w.log2_bs,
                        sh.segs, sh.wpg, wk.sq, wk.eps);
   else
-    hipLaunchKernelGGL((DecodeFragKernel<HAS_ZP, SPB, U, kWin, false, TOKS>), grid, block, 0, s, w.Bp,
-                       w.Sd, w.Zd, wk.img, wk.exps, Y, wk.P, H, bias, m, n, k, nb, w.log2_bs,
+    hipLaunchKernelGGL((DecodeFragKernel<HAS_ZP, SPB, U, kWin, false, TOKS, G, SPLIT>), grid, block, 0, s, w.Bp,
+                       w.Sd, w.Zd, wk.img, wk.exps, wk.A, Y, wk.P, H, bias, m, n, k, nb, w.log2_bs,
                        sh.segs, sh.wpg, nullptr, 0.0f);
   return hipGetLastError();
+}
+
+template <bool HAS_ZP, int SPB, int U, int TOKS>
+hipError_t LaunchMain(const WeightView &w, int64_t M, const Work &wk, float *Y, float *H,
+                      const float *bias, const Shape &sh, hipStream_t s) {
+  if constexpr (U == 1) {
+    if (wk.A != nullptr)
+      return LaunchMainG<HAS_ZP, SPB, U, TOKS, 1, true>(w, M, wk, Y, H, bias, sh, s);
+  }
+  if constexpr (TOKS == 16) {
+    if (GroupPairs(w, sh))
+      return LaunchMainG<HAS_ZP, SPB, U, TOKS, 2, false>(w, M, wk, Y, H, bias, sh, s);
+  }
+  return LaunchMainG<HAS_ZP, SPB, U, TOKS, 1, false>(w, M, wk, Y, H, bias, sh, s);
 }
 
 template <bool HAS_ZP, int SPB>
@@ -612,7 +743,10 @@ hipError_t LaunchDecodeFrag(const WeightView &w, int64_t M, const float *A, floa
   // up to 8 rows: both terms of a token in one MFMA operand (half the image)
   const bool t8 = M <= 8;
   const dim3 sgrid(static_cast<unsigned>(units * (t8 ? 4 : 8))), sblock(64);
-  if (gamma != nullptr && t8)
+  const bool split = gamma == nullptr && df::SplitInKernel(w, sh);
+  if (split) {
+    // no launch: the main kernel splits the activations itself
+  } else if (gamma != nullptr && t8)
     hipLaunchKernelGGL((df::SplitActKernel<true, 8>), sgrid, sblock, 0, s, A, img, exps, sq, gamma,
                        static_cast<int>(M), static_cast<int>(w.K));
   else if (gamma != nullptr)
@@ -629,7 +763,7 @@ hipError_t LaunchDecodeFrag(const WeightView &w, int64_t M, const float *A, floa
   // One run per group: the kernel writes Y (or H) itself and adds the bias.
   float *Hk = sh.segs == 1 ? H : nullptr;
   const float *bk = sh.segs == 1 ? bias : nullptr;
-  const df::Work wk{img, exps, gamma != nullptr ? sq : nullptr, P, eps};
+  const df::Work wk{img, exps, gamma != nullptr ? sq : nullptr, split ? A : nullptr, P, eps};
   e = w.has_zp ? df::LaunchZp<true>(w, M, wk, Y, Hk, bk, sh, s)
                       : df::LaunchZp<false>(w, M, wk, Y, Hk, bk, sh, s);
   if (e != hipSuccess || sh.segs == 1) return e;
