@@ -811,7 +811,7 @@ constexpr int kPOps0 = kPAU / kPThreads + 2;          // copies per k-tile, wave
 constexpr int kPOps1 = kPAU / kPThreads + 1;          // wavefronts 4-7 (no scale copy)
 // Cache policy of the output stores: non-temporal. Y is not read again by
 // this kernel; streaming it out keeps the L2 for the operand tiles (measured:
-// c5 gate+up M = 2048, 224 MiB of Y, 472 -> 445 us; c4 unchanged). With K
+// K = 1536, N = 14336, M = 8192, 448 MiB of Y, 443 -> 410 us; c4 unchanged). With K
 // split, the split reduction reads Y and the partial sums straight back, and
 // plain stores serve it better (c4 and c5 o at M = 512, 4 splits: 37.1 ->
 // 35.4 and 38.0 -> 36.3 us per call; qkv at M = 256 33.2 -> 32.2).
@@ -986,6 +986,22 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
         xb[(q * 4 + j) * 64 + lane] = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]),
                                                  __float_as_uint(v[2]), __float_as_uint(v[3]));
       }
+    // The exponents and the bias, all loaded here, behind the exchange:
+    // between the stores each load waited out the stores before it (M = 512,
+    // K = 14336, N = 4096 79.2 -> 76.5 us, M = 200, N = 28672 67.2 -> 64.7).
+    int er[4];
+    int4 ec[4];
+    float4 bv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) er[q] = row_exp[m0 + (4 * S + q) * 16 + (lane & 15)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int nc = min(nl + 16 * j, N - 4);
+      ec[j] = *reinterpret_cast<const int4 *>(col_exp + nc);
+      bv[j] = bias != nullptr && split == 0
+                  ? make_float4(bias[nc], bias[nc + 1], bias[nc + 2], bias[nc + 3])
+                  : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     __syncthreads();
     const uint4 *pb = lds + (wave ^ 4) * 1024;  // the partner's fragments for my rows
 #pragma unroll
@@ -1003,9 +1019,6 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
     // columns n0 + 64 cg + 16j + 4(l >> 4) + v. The accumulators are in units
     // of 2^(f_m + e_n): one ldexp per element undoes both. Split 0 writes Y
     // (and adds the bias), split s > 0 its partial sum.
-    int er[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) er[q] = row_exp[m0 + (4 * S + q) * 16 + (lane & 15)];
     if (H != nullptr) {
       const int half_n = N >> 1;
       const auto hr = __builtin_amdgcn_make_buffer_rsrc(H + static_cast<size_t>(m0) * half_n, 0,
@@ -1013,17 +1026,14 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int n = nl + 16 * j;
-        const int nc = min(n, N - 4);
-        const int e0 = col_exp[nc], e1 = col_exp[nc + 1], e2 = col_exp[nc + 2],
-                  e3 = col_exp[nc + 3];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const floatx4 a = acc[4 * S + q][j];
           const float x0 = a[0], x1 = a[1], x2 = a[2], x3 = a[3];
-          const float h0 = SiluMul(__builtin_amdgcn_ldexpf(x0, -(er[q] + e0)),
-                                   __builtin_amdgcn_ldexpf(x1, -(er[q] + e1)));
-          const float h1 = SiluMul(__builtin_amdgcn_ldexpf(x2, -(er[q] + e2)),
-                                   __builtin_amdgcn_ldexpf(x3, -(er[q] + e3)));
+          const float h0 = SiluMul(__builtin_amdgcn_ldexpf(x0, -(er[q] + ec[j].x)),
+                                   __builtin_amdgcn_ldexpf(x1, -(er[q] + ec[j].y)));
+          const float h1 = SiluMul(__builtin_amdgcn_ldexpf(x2, -(er[q] + ec[j].z)),
+                                   __builtin_amdgcn_ldexpf(x3, -(er[q] + ec[j].w)));
           const int row = (4 * S + q) * 16 + (lane & 15);
           const int off = n < N ? (row * half_n + (n >> 1)) * 4 : 0x7FFFFFF0;
           // H columns n / 2 and n / 2 + 1 are adjacent: one 8-byte store. (A
@@ -1041,24 +1051,15 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = nl + 16 * j;
-      const int nc = min(n, N - 4);
-      const int e0 = col_exp[nc], e1 = col_exp[nc + 1], e2 = col_exp[nc + 2], e3 = col_exp[nc + 3];
-      float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
-      if (bias != nullptr && split == 0) {
-        b0 = bias[nc];
-        b1 = bias[nc + 1];
-        b2 = bias[nc + 2];
-        b3 = bias[nc + 3];
-      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const floatx4 a = acc[4 * S + q][j];
         const float x0 = a[0], x1 = a[1], x2 = a[2], x3 = a[3];
         typedef unsigned int u32x4 __attribute__((vector_size(16)));
-        const u32x4 v = {__float_as_uint(__builtin_amdgcn_ldexpf(x0, -(er[q] + e0)) + b0),
-                         __float_as_uint(__builtin_amdgcn_ldexpf(x1, -(er[q] + e1)) + b1),
-                         __float_as_uint(__builtin_amdgcn_ldexpf(x2, -(er[q] + e2)) + b2),
-                         __float_as_uint(__builtin_amdgcn_ldexpf(x3, -(er[q] + e3)) + b3)};
+        const u32x4 v = {__float_as_uint(__builtin_amdgcn_ldexpf(x0, -(er[q] + ec[j].x)) + bv[j].x),
+                         __float_as_uint(__builtin_amdgcn_ldexpf(x1, -(er[q] + ec[j].y)) + bv[j].y),
+                         __float_as_uint(__builtin_amdgcn_ldexpf(x2, -(er[q] + ec[j].z)) + bv[j].z),
+                         __float_as_uint(__builtin_amdgcn_ldexpf(x3, -(er[q] + ec[j].w)) + bv[j].w)};
         const int row = (4 * S + q) * 16 + (lane & 15);
         const int off = n < N ? (row * N + n) * 4 : 0x7FFFFFF0;
         if (kt_per_split < K / kBK)  // split K: read back by the reduction
