@@ -748,16 +748,17 @@ static bool Fp32ActivationsOnly(const mnb_plan *plan) { return plan->desc.accura
 //   takes longer than this route's three launches: its time grows by about
 //   4.5 ns per M K, and with N past the 8192 wavefronts the chip holds
 //   (graph replay, us, GenericKernel against this: K = 300, N = 4000 M = 4
-//   10.7 / 11.4, M = 8 19.1 / 11.4; K = 1003, N = 4000 M = 1 8.5 / 13.2,
-//   M = 2 14.5 / 13.2; K = 1003, N = 12000 M = 1 17.8 / 13.3; K = 2500,
-//   N = 500 M = 1 13.2 / 13.5; K = 2500, N = 5001 M = 333 6350 / 45).
+//   10.7 / 11.4, M = 8 19.1 / 11.4; K = 490, N = 1157 M = 6 16.4 / 11.1;
+//   K = 2600 / 2900, N = 500 M = 1 14.1 / 15.1, 15.2 / 13.2; K = 1003 M = 1,
+//   N = 8200 / 9000 / 12000 12.8 / 13.2, 14.3 / 13.2, 16.6 / 13.1; K = 700,
+//   N = 12000 M = 1 12.3 / 13.3; K = 2500, N = 5001 M = 333 6350 / 45).
 // A launch takes at most kExactMaxRows rows (its image is then at most 1.5
 // KiB per unit and row), fewer where the workspace is smaller.
 constexpr int64_t kExactMaxRows = 2048;
 
 static bool ExactBeatsGeneric(const mnb_plan *plan, int64_t M) {
   const int64_t mk = M * plan->view.K;
-  return mk >= 2400 || mk * plan->view.N >= 8000000;
+  return mk >= 2800 || mk * plan->view.N >= 9000000;
 }
 
 static int64_t ExactRows(const mnb_plan *plan, int64_t M, int path, size_t work_bytes) {

@@ -25,8 +25,8 @@ def _plan(pkg, K, N, bs, zp, seed, level=0):
 
 
 @pytest.mark.parametrize("K,N,bs,zp,M", [
-    (2401, 1, 32, True, 1),        # one column; K one past a step
-    (65, 257, 32, False, 40),      # second 64-k tile of one value; one column past the tile
+    (2817, 1, 32, True, 1),        # one column; K one past a step
+    (65, 257, 32, False, 44),      # second 64-k tile of one value; one column past the tile
     (255, 255, 64, True, 16),      # a unit less one value; a full row tile of 16
     (257, 256, 128, True, 17),     # a second unit of one value; one row past the tile
     (1000, 300, 256, False, 31),   # blocks of a whole unit
