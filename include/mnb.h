@@ -250,7 +250,7 @@ int mnb_select_path(const mnb_plan *plan, int64_t M, int *path);
 #define MNB_KERNEL_GEMV_FRAG 10  /* GemvFragKernel: M <= 4, fp16 MFMA on nibble subnormals, fragment-ordered copy, A staged in LDS */
 
 /* Name of the main kernel mnb_run launches for M rows given workspace_bytes
- * of workspace ("GemvM1Kernel", "DecodeFragKernel", "PrefillKernel", ...;
+ * of workspace ("GemvM1Kernel", "DecodeFragKernel", "WideKernel", ...;
  * "" for M == 0 or a bad plan). Static storage. The counterpart of the
  * reference's record of the kernels a run dispatched to
  * (onnx_light_cpu/_register.py:157-170, used_kernel_names), answered before
