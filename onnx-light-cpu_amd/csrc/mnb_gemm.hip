@@ -1656,12 +1656,17 @@ size_t PrefillPartialBytes(const WeightView &w, int64_t M) {
 // 32 rows: from 16 Mi weights; smaller ones stay with GemmKernel, whose route
 // the tests fix (K = 11008, N = 1024 at M = 33 / 64 streamed 12.6 / 13.7
 // against 16.3 / 16.9 us; N = 2048 14.6 / 16.4 against 18.2 / 19.3, N = 4096
-// 21.0 / 23.0 against 25.2 / 26.9).
+// 21.0 / 23.0 against 25.2 / 26.9), and with at most an eighth of the
+// segments' steps past K (K = 2816, two segments of 64 steps for 88: N = 20480
+// at M = 45 32.4 streamed, 28.4 by GemmKernel).
 bool StreamSupportsM(const WeightView &w, int64_t M) {
   if (M < 17 || M > 64 || !PrefillSupportsShape(w) || w.K > (int64_t{1} << 22)) return false;
   if (StreamCrowded(w, M)) return false;
   const StreamShape sh = PickStreamShape(w, M, 0, 0);
-  return sh.segs > 0 && (!sh.ragged || M <= 32 || w.K * w.N >= (int64_t{16} << 20));
+  const int64_t T = w.K / 32;
+  const bool even = !sh.ragged || (int64_t{sh.segs} * sh.wpg * sh.spw - T) * 8 <= T;
+  return sh.segs > 0 &&
+         (!sh.ragged || M <= 32 || (even && w.K * w.N >= (int64_t{16} << 20)));
 }
 
 size_t StreamPartialBytes(const WeightView &w, int64_t M, int segs) {
