@@ -1108,8 +1108,8 @@ constexpr int kSGroupRows = 64;
 // StreamConverts): it loads A's fp32 values for its SPW steps first (L2-
 // resident, ahead of the weights), reduces each row's largest magnitude over
 // its own k range across the four lanes that hold the row, scales by 2^f and
-// rounds to fp16 as ConvertAKernel does, and scales its tiles by 2^-f before
-// the wavefronts' tiles meet. A finer exponent than the row's, so the
+// rounds to fp16 as ConvertAKernel does, and undoes f (with the column's exponent)
+// before the wavefronts' tiles meet. A finer exponent than the row's, so the
 // operands are ConvertAKernel's except where those fall into fp16
 // subnormals.
 template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
@@ -1190,28 +1190,34 @@ __global__ __launch_bounds__(512) void StreamKernel(
   for (int i = 0; i < WIN && i < SPW; ++i) issue(i);
   // The epilogue finishes, group by group and half by half (kHalf fragments
   // (tg, j) with j / 2 == half), fragments x = wave, wave + wpg, ... of each
-  // (wpg >= 4). Their exponents and bias are loaded behind the first weights so
-  // that their latency hides under the main loop (with two groups, whose
-  // registers they would take, in the epilogue).
+  // (wpg >= 4). The columns' exponents and the fragments' bias are loaded behind
+  // the first weights so that their latency hides under the main loop (with two
+  // groups, whose registers they would take, in the epilogue).
   constexpr int kHalf = 2 * TG;
   constexpr int kHalfItems = (kHalf + 3) / 4;
   constexpr int kMaxItems = 2 * G * kHalfItems;
   constexpr bool kPreload = G == 1;
-  int4 ec[kMaxItems];
+  int4 ec[4 * G];  // [group, j]: this lane's columns of every fragment
   float4 bv[kMaxItems];
+  auto ec_load = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < 4 * G; ++y)
+      ec[y] = *reinterpret_cast<const int4 *>(
+          col_exp + min(kSGroupRows * g + 16 * y + 4 * (lane >> 4), N - 4));
+  };
   auto item_col = [&](int it) {
     const int x = min(wave + it % kHalfItems * wpg, kHalf - 1), ph = it / kHalfItems;
     return kSGroupRows * (g + ph / 2) + 16 * (2 * (ph & 1) + (x & 1)) + 4 * (lane >> 4);
   };
-  auto item_load = [&](int it) __attribute__((always_inline)) {
+  auto item_bias = [&](int it) __attribute__((always_inline)) {
     const int nc = min(item_col(it), N - 4);
-    ec[it] = *reinterpret_cast<const int4 *>(col_exp + nc);
     bv[it] = bias != nullptr ? make_float4(bias[nc], bias[nc + 1], bias[nc + 2], bias[nc + 3])
                              : make_float4(0.f, 0.f, 0.f, 0.f);
   };
   if constexpr (kPreload) {
+    ec_load();
 #pragma unroll
-    for (int it = 0; it < kMaxItems; ++it) item_load(it);
+    for (int it = 0; it < kMaxItems; ++it) item_bias(it);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -1284,7 +1290,10 @@ __global__ __launch_bounds__(512) void StreamKernel(
     if (i + WIN < SPW) issue(i + WIN);
     __builtin_amdgcn_sched_barrier(0);
   }
-  // RMSNorm input: each row's 1 / rms from the chunks' sums of squares.
+  if constexpr (!kPreload) ec_load();
+  // RMSNorm input: each row's 1 / rms from the chunks' sums of squares, as a
+  // factor in [0.5, 1) (0 and infinity themselves) and a power of two that
+  // joins the exponents.
   float inv[TG];
 #pragma unroll
   for (int tg = 0; tg < TG; ++tg) inv[tg] = 1.0f;
@@ -1293,7 +1302,9 @@ __global__ __launch_bounds__(512) void StreamKernel(
     for (int tg = 0; tg < TG; ++tg) {
       float q = 0.0f;
       for (int ch = 0; ch * kChunkK < K; ++ch) q += sq[ch * 16 * TG + 16 * tg + (lane & 15)];
-      inv[tg] = 1.0f / sqrtf(q / static_cast<float>(K) + eps);
+      const float r = 1.0f / sqrtf(q / static_cast<float>(K) + eps);
+      inv[tg] = __builtin_amdgcn_frexp_mantf(r);
+      fw[tg] -= __builtin_amdgcn_frexp_expf(r);
     }
   }
 
@@ -1303,7 +1314,9 @@ __global__ __launch_bounds__(512) void StreamKernel(
   // wavefronts' tiles in wavefront order. Lane l holds row 16 tg + (l & 15)
   // and the 4 columns 64 g + 16 j + 4 (l >> 4) .. + 3. A wavefront past K
   // (the end of a shorter last segment) ran on loads beyond the weights'
-  // buffers (zeros) and activations past its rows: it adds nothing.
+  // buffers (zeros) and activations past its rows: it adds nothing. The row's
+  // and the column's exponent are undone together: the sums are products times
+  // 2^(f + e), and undoing f alone leaves large rows beyond fp32.
   const bool past_k = s0 >= T;
   float *out = seg == 0 ? Y : partials + static_cast<size_t>(seg - 1) * M * N;
 #pragma unroll
@@ -1315,8 +1328,11 @@ __global__ __launch_bounds__(512) void StreamKernel(
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         floatx4 t = acc[ph / 2][tg][2 * half + jj];
+        const int4 e4 = ec[2 * ph + jj];
+        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) t[q] = __builtin_amdgcn_ldexpf(t[q], -fw[tg]) * inv[tg];
+        for (int q = 0; q < 4; ++q)
+          t[q] = __builtin_amdgcn_ldexpf(t[q] * inv[tg], -(fw[tg] + ev[q]));
         sred[(wave * kHalf + tg * 2 + jj) * 64 + lane] = past_k ? floatx4{0.f, 0.f, 0.f, 0.f} : t;
       }
     __syncthreads();
@@ -1325,15 +1341,11 @@ __global__ __launch_bounds__(512) void StreamKernel(
       const int x = wave + hi * wpg;
       if (x >= kHalf) break;
       const int it = ph * kHalfItems + hi;
-      if constexpr (!kPreload) item_load(it);
-      floatx4 sum = sred[x * 64 + lane];
-      for (int w = 1; w < wpg; ++w) sum += sred[(w * kHalf + x) * 64 + lane];
+      if constexpr (!kPreload) item_bias(it);
+      floatx4 v = sred[x * 64 + lane];
+      for (int w = 1; w < wpg; ++w) v += sred[(w * kHalf + x) * 64 + lane];
       const int m = 16 * (x >> 1) + (lane & 15);
       const int n = item_col(it);
-      const int ecv[4] = {ec[it].x, ec[it].y, ec[it].z, ec[it].w};
-      floatx4 v;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = __builtin_amdgcn_ldexpf(sum[q], -ecv[q]);
       const bool ok = m < M && n < N;
       if (H != nullptr) {
         // gate/up pairs (columns n, n + 1 and n + 2, n + 3): H columns n / 2, n / 2 + 1

@@ -254,3 +254,43 @@ def test_stream_shapes_rms_and_bias(pkg, orc, cuda, K, N, bs, zp, M):
         if n64[i].any():
             assert orc.l2_rel_error(Yn[i:i + 1, cols], n64[i:i + 1]) <= 2e-3, keep[i]
     op.release()
+
+
+@pytest.mark.parametrize("K,N,bs,zp,M", [
+    (4096, 4096, 128, False, 32),  # the wavefronts convert the activations; four segments
+    (512, 64, 32, True, 40),       # the image, one group, one segment
+    (4096, 28672, 128, True, 48),  # two column groups, one segment
+    (14336, 4096, 128, True, 64),  # two column groups, several segments
+])
+def test_stream_largest_magnitudes(pkg, orc, cuda, K, N, bs, zp, M):
+    """Rows near both ends of fp32: 1e36 times N(0, 1) gives outputs of up to
+    5e37 here, finite in fp32, and must stay so although the kernel's sums are
+    scaled (by 2^17 at these weight scales, until the column exponent is
+    undone). The GEMM's bound row by row. RMSNorm rows whose squares overflow
+    have 1 / rms = 0 in fp32, and zero outputs."""
+    import torch
+    p = pkg.workloads.Projection("range", K, N, bs, zp)
+    B, S, Z = pkg.workloads.make_weights(p, K + N + 1)
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare(B, S, Z)
+    A = pkg.workloads.make_activations(M, K, 1.0, M + 1)
+    A[1] *= 1e33
+    A[2] *= 1e36
+    A[3, :] *= 1e-33
+    A[M - 1] *= 1e36
+    rng = np.random.default_rng(N + 1)
+    cols = np.unique(np.concatenate([rng.integers(0, N, 96), [0, N - 1]]))
+    print(f"case stream largest magnitudes K={K} N={N} M={M} kernel={op.kernel_name(M)}",
+          flush=True)
+    assert op.kernel_name(M) == "StreamKernel"
+    dA = torch.from_numpy(A).to(cuda)
+    y64 = orc.matmul_nbits_f64(A, B[cols], S[cols], None if Z is None else Z[cols], K, len(cols), bs)
+    assert np.abs(y64).max() < 3e38
+    Y = op(dA).cpu().numpy()
+    Yn = op.run_rmsnorm(dA, torch.ones(K, device=cuda), 1e-5).cpu().numpy()
+    op.release()
+    assert np.isfinite(Y).all()
+    for m in range(M):
+        assert orc.l2_rel_error(Y[m:m + 1, cols], y64[m:m + 1]) <= GEMM_TOL, m
+    assert np.isfinite(Yn).all()
+    for m in (1, 2, M - 1):
+        assert not Yn[m].any(), m
