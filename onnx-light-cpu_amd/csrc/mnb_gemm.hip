@@ -167,93 +167,79 @@ __global__ __launch_bounds__(256) void ConvertAKernel(const float *__restrict__ 
   }
 }
 
-// StreamKernel's conversion of A: one workgroup of 8 wavefronts per (chunk of
-// kChunkK k, group of 16 rows), wavefront w its steps 2 w and 2 w + 1, lane l
-// 8 k of row l & 15 per step. Each row's chunk is scaled by 2^f, f =
-// RangeExponent of the chunk's largest magnitude (StreamKernel's wavefronts
-// stay inside one chunk and undo f in their sums), rounded to fp16 as
-// ConvertAKernel does and written as 1 KiB operand records, the lanes
-// contiguous: no row-wide reduction, whole cache lines per store. With gamma
-// (RMSNorm folded in) the values are x * gamma and sq receives each row's sum
-// of x^2 over the chunk, from which StreamKernel forms 1 / rms.
+// StreamKernel's conversion of A: one workgroup of 4 wavefronts per (chunk of
+// kChunkK k, kChunkRows rows), a thread 8 k of one row. Each row's chunk is
+// scaled by 2^f, f = RangeExponent of the chunk's largest magnitude
+// (StreamKernel's wavefronts stay inside one chunk and undo f in their sums),
+// rounded to fp16 as ConvertAKernel does and written into 1 KiB operand records
+// of 16 rows: no row-wide reduction. With gamma (RMSNorm folded in) the values
+// are x * gamma and sq receives each row's sum of x^2 over the chunk, from which
+// StreamKernel forms 1 / rms. A CU reads and writes kChunkRows x 3 KiB: with 16
+// rows per workgroup a few CUs had four times that to do (K = 4096
+// at M = 33 to 48 3.5 us, now 2.9).
+constexpr int kChunkRows = 4;
 constexpr int kChunkK = 512;
 template <bool RMS>
-__global__ __launch_bounds__(512) void ConvertChunkKernel(const float *__restrict__ A,
+__global__ __launch_bounds__(256) void ConvertChunkKernel(const float *__restrict__ A,
                                                           uint4 *__restrict__ img,
                                                           int *__restrict__ exps,
                                                           float *__restrict__ sq,
                                                           const float *__restrict__ gamma, int M,
                                                           int K, int chunks, int rows_padded) {
-  __shared__ float red[8][16], reds[RMS ? 8 : 1][16];
+  __shared__ float red[4][kChunkRows], reds[RMS ? 4 : 1][kChunkRows];
   const int ch = static_cast<int>(blockIdx.x) % chunks;
-  const int mt = static_cast<int>(blockIdx.x) / chunks;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15;
+  const int m0 = static_cast<int>(blockIdx.x) / chunks * kChunkRows;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int r = tid % kChunkRows, unit = tid / kChunkRows;
   const int T = K / 32;
-  const int rows = min(16, M - 16 * mt);
-  const int bytes = rows * K * 4;
+  const int s = ch * (kChunkK / 32) + unit / 4;
+  const int rows = min(kChunkRows, M - m0);  // <= 0: padding rows, zeros
+  const int bytes = max(rows, 0) * K * 4;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float *>(A + static_cast<size_t>(16 * mt) * K), 0, bytes, 0x00020000);
-  floatx4 x[2][2], gm[2][2];
-  float amax = 0.0f;
+      const_cast<float *>(A + static_cast<size_t>(min(m0, M - 1)) * K), 0, bytes, 0x00020000);
+  // rows past M and steps past K read beyond the buffer: zeros
+  const int k = 32 * s + 8 * (unit % 4);
+  const int vo = r < rows && s < T ? (r * K + k) * 4 : bytes;
+  floatx4 x[2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    // rows past M and steps past K read beyond the buffer: zeros
-    const int s = ch * (kChunkK / 32) + 2 * wave + h;
-    const int vo = r < rows && s < T ? (r * K + 32 * s + 8 * (lane >> 4)) * 4 : bytes;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      x[h][p] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra, vo + 16 * p, 0, 0));
-      if constexpr (RMS)
-        gm[h][p] = reinterpret_cast<const floatx4 *>(gamma + 32 * min(s, T - 1) + 8 * (lane >> 4))[p];
-    }
-  }
+  for (int p = 0; p < 2; ++p)
+    x[p] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(ra, vo + 16 * p, 0, 0));
   if constexpr (RMS) {
+    const floatx4 *gp = reinterpret_cast<const floatx4 *>(gamma + min(k, K - 8));
+    const floatx4 g0 = gp[0], g1 = gp[1];
     float q = 0.0f;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) q += x[h][p][v] * x[h][p][v];
-        x[h][p] *= gm[h][p];
-      }
-    q += Xor16(q);
-    q += __shfl_xor(q, 32, 64);
-    if (lane < 16) reds[wave][lane] = q;
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) amax = fmaxf(amax, fabsf(x[h][p][v]));
-  amax = fmaxf(amax, Xor16(amax));
-  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-  if (lane < 16) red[wave][lane] = amax;
+      for (int v = 0; v < 4; ++v) q += x[p][v] * x[p][v];
+    x[0] *= g0;
+    x[1] *= g1;
+#pragma unroll
+    for (int o = kChunkRows; o < 64; o *= 2) q += __shfl_xor(q, o, 64);
+    if ((tid & 63) < kChunkRows) reds[wave][r] = q;
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) amax = fmaxf(amax, fabsf(x[p][v]));
+#pragma unroll
+  for (int o = kChunkRows; o < 64; o *= 2) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  if ((tid & 63) < kChunkRows) red[wave][r] = amax;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < 8; ++w) amax = fmaxf(amax, red[w][r]);
+  for (int w = 0; w < 4; ++w) amax = fmaxf(amax, red[w][r]);
   const int f = RangeExponent(amax, kRowExpTarget);
-  if (threadIdx.x < 16) {
-    exps[ch * rows_padded + 16 * mt + lane] = f;
-    if constexpr (RMS) {
-      float q = 0.0f;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) q += reds[w][lane];
-      sq[ch * rows_padded + 16 * mt + lane] = q;
-    }
+  if (tid < kChunkRows) {
+    exps[ch * rows_padded + m0 + r] = f;
+    if constexpr (RMS)
+      sq[ch * rows_padded + m0 + r] = (reds[0][r] + reds[1][r]) + (reds[2][r] + reds[3][r]);
   }
   auto sc = [f](float v) { return __builtin_amdgcn_ldexpf(v, f); };
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int s = ch * (kChunkK / 32) + 2 * wave + h;
-    const floatx4 a = x[h][0], b = x[h][1];
-    if (s < T)
-      img[(static_cast<size_t>(mt) * T + s) * 64 + lane] =
-          make_uint4(PackHalf2(sc(a[0]), sc(b[0])), PackHalf2(sc(a[1]), sc(b[1])),
-                     PackHalf2(sc(a[2]), sc(b[2])), PackHalf2(sc(a[3]), sc(b[3])));
-  }
+  if (s < T)
+    img[(static_cast<size_t>(m0 / 16) * T + s) * 64 + 16 * (unit % 4) + m0 % 16 + r] =
+        make_uint4(PackHalf2(sc(x[0][0]), sc(x[1][0])), PackHalf2(sc(x[0][1]), sc(x[1][1])),
+                   PackHalf2(sc(x[0][2]), sc(x[1][2])), PackHalf2(sc(x[0][3]), sc(x[1][3])));
 }
 
 // One k-tile of B for this thread: 32 nibbles of one weight row (one
@@ -1101,6 +1087,12 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
 // step beside 1.25 KiB of weights, from the L2) bound the kernel (K = 4096,
 // N = 28672, 448 groups: M = 48 / 64 30.4 / 34.0 -> 27.3 / 29.8 us).
 constexpr int kSGroupRows = 64;
+// PARTS: in how many parts a group's tiles meet in LDS. All at once (4 TG KiB
+// per wavefront) saves barriers and lets every wavefront of eight finish a
+// fragment (K = N = 4096 at M = 17 8.6 -> 8.1 us); with more than two row tiles
+// and more than four wavefronts in two parts, so that two workgroups fit a CU.
+template <int TG, int G>
+constexpr int StreamParts(int wpg) { return G == 1 && (TG == 2 || wpg == 4) ? 1 : 2; }
 
 //
 // CVT: the wavefront converts its own activations instead of reading the
@@ -1112,14 +1104,15 @@ constexpr int kSGroupRows = 64;
 // before the wavefronts' tiles meet. A finer exponent than the row's, so the
 // operands are ConvertAKernel's except where those fall into fp16
 // subnormals.
-template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
+template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G, int PARTS>
 __global__ __launch_bounds__(512) void StreamKernel(
     const uint4 *__restrict__ Ah, const float *__restrict__ A, const uint8_t *__restrict__ Bp,
     const uint8_t *__restrict__ Sp, float *__restrict__ Y, float *__restrict__ partials,
     float *__restrict__ H, const int *__restrict__ row_exp, const int *__restrict__ col_exp,
     const float *__restrict__ bias, const float *__restrict__ sq, float eps, int M, int N, int K,
     int log2_bs, int segs, int wpg) {
-  extern __shared__ floatx4 sred[];  // [wave][2 tg + (j & 1)][lane], j / 2 one half
+  extern __shared__ floatx4 sred[];  // [wave][kJ tg + j % kJ][lane], one part of the fragments
+  __shared__ float qs[CVT ? 1 : 8][TG][16], rms_inv[CVT ? 1 : 8][16 * TG];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int g = static_cast<int>(blockIdx.x) / segs * G;  // first group
@@ -1186,28 +1179,45 @@ __global__ __launch_bounds__(512) void StreamKernel(
                                                  ra, (tg * T + s) * 1024 + 16 * lane, 0, 0));
     }
   };
-#pragma unroll
-  for (int i = 0; i < WIN && i < SPW; ++i) issue(i);
-  // The epilogue finishes, group by group and half by half (kHalf fragments
-  // (tg, j) with j / 2 == half), fragments x = wave, wave + wpg, ... of each
-  // (wpg >= 4). The columns' exponents and the fragments' bias are loaded behind
-  // the first weights so that their latency hides under the main loop (with two
-  // groups, whose registers they would take, in the epilogue).
-  constexpr int kHalf = 2 * TG;
-  constexpr int kHalfItems = (kHalf + 3) / 4;
-  constexpr int kMaxItems = 2 * G * kHalfItems;
+  // The columns' exponents come ahead of the weights and the epilogue's bias
+  // behind the first of them, so that their latency hides under the main loop
+  // (with two groups, whose registers they would take, in the epilogue).
   constexpr bool kPreload = G == 1;
   int4 ec[4 * G];  // [group, j]: this lane's columns of every fragment
-  float4 bv[kMaxItems];
   auto ec_load = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int y = 0; y < 4 * G; ++y)
       ec[y] = *reinterpret_cast<const int4 *>(
           col_exp + min(kSGroupRows * g + 16 * y + 4 * (lane >> 4), N - 4));
   };
+  if constexpr (kPreload) ec_load();
+  // RMSNorm input: this wavefront's part of each row's sum of squares, chunks
+  // 4 wave + (lane >> 4), + 4 wpg, ... (64 TG bytes each, zeros past the last).
+  // Loaded ahead of the weights and added while those are on their way: every
+  // wavefront adding all of them after the main loop took 1 to 2 us more.
+  const int sq_bytes = CVT || sq == nullptr ? 0 : (K + kChunkK - 1) / kChunkK * 64 * TG;
+  const int sq_off = (4 * wave + (lane >> 4)) * 64 * TG + 4 * (lane & 15);
+  const int sq_step = 4 * wpg * 64 * TG;
+  const __amdgpu_buffer_rsrc_t rq =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(sq), 0, sq_bytes, 0x00020000);
+  float sqv[TG];
+  if constexpr (!CVT) {
+#pragma unroll
+    for (int tg = 0; tg < TG; ++tg)
+      sqv[tg] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rq, sq_off + 64 * tg, 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < WIN && i < SPW; ++i) issue(i);
+  // The epilogue finishes, group by group, PARTS parts of the fragments (tg, j)
+  // (part j / kJ, kPart fragments), x = wave, wave + wpg, ... of each (wpg >= 4).
+  constexpr int kJ = 4 / PARTS;
+  constexpr int kPart = kJ * TG;
+  constexpr int kPartItems = (kPart + 3) / 4;
+  constexpr int kMaxItems = PARTS * G * kPartItems;
+  float4 bv[kMaxItems];
   auto item_col = [&](int it) {
-    const int x = min(wave + it % kHalfItems * wpg, kHalf - 1), ph = it / kHalfItems;
-    return kSGroupRows * (g + ph / 2) + 16 * (2 * (ph & 1) + (x & 1)) + 4 * (lane >> 4);
+    const int x = min(wave + it % kPartItems * wpg, kPart - 1), ph = it / kPartItems;
+    return kSGroupRows * g + 16 * (kJ * ph + x % kJ) + 4 * (lane >> 4);
   };
   auto item_bias = [&](int it) __attribute__((always_inline)) {
     const int nc = min(item_col(it), N - 4);
@@ -1215,11 +1225,28 @@ __global__ __launch_bounds__(512) void StreamKernel(
                              : make_float4(0.f, 0.f, 0.f, 0.f);
   };
   if constexpr (kPreload) {
-    ec_load();
 #pragma unroll
     for (int it = 0; it < kMaxItems; ++it) item_bias(it);
   }
   __builtin_amdgcn_sched_barrier(0);
+
+  if (!CVT && sq != nullptr) {
+#pragma unroll
+    for (int tg = 0; tg < TG; ++tg) {
+      for (int o = sq_off + sq_step; o < sq_bytes; o += sq_step)
+        sqv[tg] += __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rq, o + 64 * tg, 0, 0));
+      float q = sqv[tg];
+      q += Xor16(q);
+      q += __shfl_xor(q, 32, 64);
+      if (lane < 16) qs[wave][tg][lane] = q;
+    }
+    __syncthreads();
+    // row `lane`'s 1 / rms, kept for this wavefront's epilogue
+    const int rl = min(lane, 16 * TG - 1);
+    float q = 0.0f;
+    for (int w = 0; w < wpg; ++w) q += qs[w][rl / 16][rl % 16];
+    if (lane < 16 * TG) rms_inv[wave][lane] = 1.0f / sqrtf(q / static_cast<float>(K) + eps);
+  }
 
   // CVT: each row's exponent over this wavefront's k range (the row's values
   // sit in lanes r, r + 16, r + 32, r + 48), then the fp16 fragments.
@@ -1291,26 +1318,22 @@ __global__ __launch_bounds__(512) void StreamKernel(
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (!kPreload) ec_load();
-  // RMSNorm input: each row's 1 / rms from the chunks' sums of squares, as a
-  // factor in [0.5, 1) (0 and infinity themselves) and a power of two that
-  // joins the exponents.
+  // RMSNorm input: each row's 1 / rms as a factor in [0.5, 1) (0 and infinity
+  // themselves) and a power of two that joins the exponents.
   float inv[TG];
 #pragma unroll
   for (int tg = 0; tg < TG; ++tg) inv[tg] = 1.0f;
-  if (sq != nullptr) {
+  if (!CVT && sq != nullptr) {
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg) {
-      float q = 0.0f;
-      for (int ch = 0; ch * kChunkK < K; ++ch) q += sq[ch * 16 * TG + 16 * tg + (lane & 15)];
-      const float r = 1.0f / sqrtf(q / static_cast<float>(K) + eps);
+      const float r = rms_inv[wave][16 * tg + (lane & 15)];
       inv[tg] = __builtin_amdgcn_frexp_mantf(r);
       fw[tg] -= __builtin_amdgcn_frexp_expf(r);
     }
   }
 
-  // The wavefronts' tiles meet in LDS, half the fragments (j = 0, 1, then 2,
-  // 3) at a time so that two workgroups fit a CU; wavefront w finishes the
-  // half's fragments x = 2 tg + (j & 1) = w, w + wpg, ..., adding the
+  // The wavefronts' tiles meet in LDS, part by part; wavefront w finishes the
+  // part's fragments x = kJ tg + j % kJ = w, w + wpg, ..., adding the
   // wavefronts' tiles in wavefront order. Lane l holds row 16 tg + (l & 15)
   // and the 4 columns 64 g + 16 j + 4 (l >> 4) .. + 3. A wavefront past K
   // (the end of a shorter last segment) ran on loads beyond the weights'
@@ -1320,31 +1343,30 @@ __global__ __launch_bounds__(512) void StreamKernel(
   const bool past_k = s0 >= T;
   float *out = seg == 0 ? Y : partials + static_cast<size_t>(seg - 1) * M * N;
 #pragma unroll
-  for (int ph = 0; ph < 2 * G; ++ph) {  // (group, half)
-    const int half = ph & 1;
+  for (int ph = 0; ph < PARTS * G; ++ph) {  // (group, part)
     if (ph > 0) __syncthreads();
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        floatx4 t = acc[ph / 2][tg][2 * half + jj];
-        const int4 e4 = ec[2 * ph + jj];
+      for (int jj = 0; jj < kJ; ++jj) {
+        floatx4 t = acc[ph / PARTS][tg][kJ * (ph % PARTS) + jj];
+        const int4 e4 = ec[kJ * ph + jj];
         const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           t[q] = __builtin_amdgcn_ldexpf(t[q] * inv[tg], -(fw[tg] + ev[q]));
-        sred[(wave * kHalf + tg * 2 + jj) * 64 + lane] = past_k ? floatx4{0.f, 0.f, 0.f, 0.f} : t;
+        sred[(wave * kPart + tg * kJ + jj) * 64 + lane] = past_k ? floatx4{0.f, 0.f, 0.f, 0.f} : t;
       }
     __syncthreads();
 #pragma unroll
-    for (int hi = 0; hi < kHalfItems; ++hi) {
+    for (int hi = 0; hi < kPartItems; ++hi) {
       const int x = wave + hi * wpg;
-      if (x >= kHalf) break;
-      const int it = ph * kHalfItems + hi;
+      if (x >= kPart) break;
+      const int it = ph * kPartItems + hi;
       if constexpr (!kPreload) item_bias(it);
       floatx4 v = sred[x * 64 + lane];
-      for (int w = 1; w < wpg; ++w) v += sred[(w * kHalf + x) * 64 + lane];
-      const int m = 16 * (x >> 1) + (lane & 15);
+      for (int w = 1; w < wpg; ++w) v += sred[(w * kPart + x) * 64 + lane];
+      const int m = 16 * (x / kJ) + (lane & 15);
       const int n = item_col(it);
       const bool ok = m < M && n < N;
       if (H != nullptr) {
@@ -1448,17 +1470,29 @@ struct StreamIn {
   float eps;
 };
 
-template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
-hipError_t LaunchStreamT(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
-                         float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
+template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G, int PARTS>
+hipError_t LaunchStreamParts(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
+                             float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
-  const size_t lds = static_cast<size_t>(sh.wpg) * TG * 2 * 64 * 16;
+  const size_t lds = static_cast<size_t>(sh.wpg) * TG * (4 / PARTS) * 64 * 16;
   const dim3 grid(static_cast<unsigned>((groups + G - 1) / G * sh.segs)), block(64 * sh.wpg);
-  hipLaunchKernelGGL((StreamKernel<HAS_ZP, TG, SPW, WIN, CVT, G>), grid, block, lds, s, in.Ah, in.A,
-                     w.Bp, w.Sp, Y, P, H, in.exps, w.col_exp, bias, in.sq, in.eps,
+  hipLaunchKernelGGL((StreamKernel<HAS_ZP, TG, SPW, WIN, CVT, G, PARTS>), grid, block, lds, s, in.Ah,
+                     in.A, w.Bp, w.Sp, Y, P, H, in.exps, w.col_exp, bias, in.sq, in.eps,
                      static_cast<int>(M), static_cast<int>(w.N), static_cast<int>(w.K), w.log2_bs,
                      sh.segs, sh.wpg);
   return hipGetLastError();
+}
+
+template <bool HAS_ZP, int TG, int SPW, int WIN, bool CVT, int G>
+hipError_t LaunchStreamT(const WeightView &w, int64_t M, const StreamIn &in, float *Y, float *P,
+                         float *H, const float *bias, const StreamShape &sh, hipStream_t s) {
+  if constexpr (StreamParts<TG, G>(4) == 1) {
+    if (StreamParts<TG, G>(sh.wpg) == 1)
+      return LaunchStreamParts<HAS_ZP, TG, SPW, WIN, CVT, G, 1>(w, M, in, Y, P, H, bias, sh, s);
+  }
+  if constexpr (StreamParts<TG, G>(8) == 2)
+    return LaunchStreamParts<HAS_ZP, TG, SPW, WIN, CVT, G, 2>(w, M, in, Y, P, H, bias, sh, s);
+  return hipErrorInvalidValue;
 }
 
 template <bool HAS_ZP, int TG>
@@ -1730,7 +1764,7 @@ hipError_t LaunchStream(const WeightView &w, int64_t M, const float *A, float *Y
     const int m = static_cast<int>(M), K = static_cast<int>(w.K);
     const int groups = static_cast<int>((M + 15) / 16), chunks = (K + kChunkK - 1) / kChunkK;
     float *sq = reinterpret_cast<float *>(exps + chunks * 16 * groups);
-    const dim3 grid(chunks * groups), block(512);
+    const dim3 grid(chunks * groups * (16 / kChunkRows)), block(256);
     if (gamma != nullptr) {
       in.sq = sq;
       hipLaunchKernelGGL(ConvertChunkKernel<true>, grid, block, 0, s, A, Ah, exps, sq, gamma, m, K,
