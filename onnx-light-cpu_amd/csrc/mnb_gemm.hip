@@ -1395,7 +1395,6 @@ __global__ __launch_bounds__(512) void StreamKernel(
 
 struct StreamShape {
   int segs, wpg, spw;
-  bool ragged = false;  // a shorter last segment
   int groups = 1;       // 64-row groups per workgroup
 };
 // Steps in flight with two groups per wavefront: 16 (w, sz) + 4 TG VGPRs each
@@ -1403,61 +1402,76 @@ struct StreamShape {
 template <int TG>
 constexpr int WinG2() { return TG == 2 ? 4 : TG == 3 ? 3 : 2; }
 
+// Whether a launch's wavefronts convert their own activations: at most 8
+// fragments per wavefront (two row tiles of 4 steps) and no more workgroups
+// than CUs. It saves the conversion's launch, 1.3 us of a call at M = 17 and 0.9
+// at M = 32 with four wavefronts per workgroup, 0.9 and nothing with eight (K =
+// 2048, N = 512 9.7 -> 8.2 and 9.8 -> 8.9 us); slower where the fragments or the
+// workgroups are more (K = N = 4096 at M = 48 / 64 +0.4 / +1.2 us, 8 steps per
+// wavefront at M = 32 +4.9 us, 1.5 workgroups per CU +1.4 us).
+inline bool StreamConverts(const WeightView &w, int64_t M, const StreamShape &sh) {
+  const int64_t wgs = (w.N + kSGroupRows - 1) / kSGroupRows * sh.segs;
+  return sh.groups == 1 && (M + 15) / 16 * sh.spw <= 8 && wgs <= w.num_cus;
+}
+
 // The launch shape: groups of 64 rows per workgroup, K segments, wavefronts
 // per workgroup (4 to 8) and steps per wavefront (4, 8 or 16; 8 or 16 with two
-// groups) with whose product K / 32 divides; only where none does, shapes whose
-// last segment is shorter. Least cost in steps of one wavefront: the rounds that the busiest CU runs
-// (one workgroup at a time) times a wavefront's steps plus 5.5 for the launch's
-// fill and drain, plus 4 for the reduction of several segments; a step of two
-// groups counts 1.75 (two row tiles) or 1.55 (more), since the activations are
-// loaded once. Fewer segments on a tie. It gives within 10% of the measured
-// times (M = 48, us: K = N = 4096 four segments of 8 x 4 12.4, two of 8 x 8
-// 13.9, one of 8 x 16 15.8; N = 6144 four of 8 x 4, 1.5 rounds, 17.7, two of
-// 8 x 8 14.4; K = 14336, N = 4096 seven of 8 x 8 24.2, four of 7 x 16 19.8;
-// N = 28672 one of 8 x 16 30.4, two groups per workgroup 27.3).
-inline StreamShape PickStreamShape(const WeightView &w, int64_t M, int segs_req, int spw_req) {
+// groups); the last segment may be shorter. The least estimated time in us, a
+// fit to 5700 measured calls (51 weights, six M, every shape; the shape taken is
+// 0.5% from the fastest on average, 10% at most): the busiest SIMD runs `waves`
+// wavefronts, each of `spw` steps, a fill and an exchange per fragment (five to
+// seven in a workgroup put two on some SIMDs; with two groups, whose registers
+// allow one workgroup per CU, they cost as eight); several segments add the
+// launch and the traffic of the reduction. Estimated by rounds of workgroups
+// times steps the shape was 7% from the fastest, and up to 40% on small
+// weights, where a step costs a memory latency. us: K = 2048, N = 512 at M =
+// 17 / 33 one segment of 8 x 8 10.2 / 12.2, four of 4 x 4 8.2 / 10.4; K = N =
+// 5120 at M = 48 two groups, four of 5 x 8 20.6, one group, three of 4 x 16 15.1;
+// K = 12288, N = 16384 at M = 17 six of 8 x 8 46.9, six of 4 x 16 35.4; K = 4096,
+// N = 28672 at M = 48 two groups, one of 8 x 16 26.3, one group 30.2.
+// M counts as the largest of its class: 24, 32, 48 or 64.
+inline StreamShape PickStreamShape(const WeightView &w, int64_t rows, int segs_req, int spw_req) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
   const int T = static_cast<int>(w.K / 32);
   if (segs_req > 0 && spw_req > 0) {
     const int per = segs_req * spw_req;
     return StreamShape{segs_req, T % per == 0 ? T / per : 0, spw_req};
   }
+  const int64_t M = rows <= 24 ? 24 : (rows + 15) / 16 * 16;
+  const int tg = static_cast<int>((M + 15) / 16);
   StreamShape best{0, 0, 0};
-  double best_cost = 0.0;
-  for (bool ragged : {false, true}) {
-    for (int g : {1, 2})
-      for (int segs = 1; segs <= kMaxSplits; ++segs)
-        for (int spw : {16, 8, 4}) {
-          if (T % spw != 0 || (g == 2 && spw == 4)) continue;
-          const int wpg = std::max(4, (T / spw + segs - 1) / segs);  // wavefronts cover a segment
-          const int per = wpg * spw;
-          if (wpg > 8 || (T + per - 1) / per != segs || (T % per != 0) != ragged) continue;
-          const int64_t wgs = (groups + g - 1) / g * segs;
-          const int64_t rounds = (wgs + w.num_cus - 1) / std::max(1, w.num_cus);
-          const double step = g == 1 ? 1.0 : M <= 32 ? 1.75 : 1.55;
-          const double cost =
-              static_cast<double>(rounds) * (spw * step + 5.5) + (segs > 1 ? 4.0 : 0.0);
-          if (best.wpg == 0 || cost < best_cost - 1e-9 ||
-              (cost < best_cost + 1e-9 && segs < best.segs)) {
-            best = StreamShape{segs, wpg, spw, ragged, g};
-            best_cost = cost;
-          }
+  double best_us = 0.0;
+  for (int g : {1, 2})
+    for (int spw : {16, 8, 4}) {
+      if (T % spw != 0 || (g == 2 && spw == 4)) continue;
+      for (int segs = 1; segs <= kMaxSplits; ++segs) {
+        const int wpg = std::max(4, (T / spw + segs - 1) / segs);  // wavefronts cover a segment
+        const int per = wpg * spw, simd = (wpg + 3) / 4;
+        if (wpg > 8 || (T + per - 1) / per != segs) continue;
+        const StreamShape sh{segs, wpg, spw, g};
+        const int64_t wgs = (groups + g - 1) / g * segs;
+        const int64_t rounds = (wgs + w.num_cus - 1) / std::max(1, w.num_cus);
+        const double waves = rounds * (g == 1 ? 0.8 * simd + 0.05 * wpg : simd);
+        double us = g == 1 ? waves * ((0.1 + 0.035 * tg) * spw + 0.25 * tg)
+                           : waves * ((0.15 + 0.04 * tg) * spw + 0.3 * tg + 1.4) + 1.3;
+        if (segs > 1) us += 1.65 + 0.05 * segs + 0.6e-6 * (segs + 1) * M * w.N;
+        if (StreamConverts(w, M, sh)) us -= M <= 24 ? 1.75 - 0.4 * simd : 1.9 - simd;
+        if (best.segs == 0 || us < best_us) {
+          best = sh;
+          best_us = us;
         }
-    if (best.wpg != 0) break;
-  }
+      }
+    }
   return best;
 }
 
-// Whether the wavefronts convert their own activations: no RMSNorm input, at
-// most 8 fragments per wavefront, and no more workgroups than CUs. Measured
-// per call against ConvertAKernel + the image: c4 M = 17 / 32 10.45 -> 8.79
-// / 10.76 -> 10.11 us; slower where the fragments or the workgroups are more
-// (c4 M = 48 / 64 +0.4 / +1.2 us, c3 M = 32 with 8 steps per wavefront
-// +4.9 us, c5 qkv M = 32 with 1.5 workgroups per CU +1.4 us), so only with
-// two row tiles and 4 steps.
-inline bool StreamConverts(const WeightView &w, int64_t M, const StreamShape &sh, bool rms) {
-  const int64_t wgs = (w.N + kSGroupRows - 1) / kSGroupRows * sh.segs;
-  return !rms && sh.groups == 1 && (M + 15) / 16 * sh.spw <= 8 && wgs <= w.num_cus;
+// Whether K / 32 steps divide evenly into such segments.
+inline bool StreamEven(const WeightView &w) {
+  const int T = static_cast<int>(w.K / 32);
+  for (int spw : {16, 8, 4})
+    for (int wpg = 4; wpg <= 8; ++wpg)
+      if (T % (wpg * spw) == 0 && T / (wpg * spw) <= kMaxSplits) return true;
+  return false;
 }
 
 // The launch's operands: the fp16 image with its chunk exponents and (RMSNorm)
@@ -1702,17 +1716,13 @@ size_t PrefillPartialBytes(const WeightView &w, int64_t M) {
 // 32 rows: from 16 Mi weights; smaller ones stay with GemmKernel, whose route
 // the tests fix (K = 11008, N = 1024 at M = 33 / 64 streamed 12.6 / 13.7
 // against 16.3 / 16.9 us; N = 2048 14.6 / 16.4 against 18.2 / 19.3, N = 4096
-// 21.0 / 23.0 against 25.2 / 26.9), and with at most an eighth of the
-// segments' steps past K (K = 2816, two segments of 64 steps for 88: N = 20480
-// at M = 45 32.4 streamed, 28.4 by GemmKernel).
+// 21.0 / 23.0 against 25.2 / 26.9; K = 2816, N = 20480 at M = 33 / 48 / 64
+// 23.0 / 24.8 / 28.9 against 26.8 / 27.9 / 28.9).
 bool StreamSupportsM(const WeightView &w, int64_t M) {
   if (M < 17 || M > 64 || !PrefillSupportsShape(w) || w.K > (int64_t{1} << 22)) return false;
   if (StreamCrowded(w, M)) return false;
-  const StreamShape sh = PickStreamShape(w, M, 0, 0);
-  const int64_t T = w.K / 32;
-  const bool even = !sh.ragged || (int64_t{sh.segs} * sh.wpg * sh.spw - T) * 8 <= T;
-  return sh.segs > 0 &&
-         (!sh.ragged || M <= 32 || (even && w.K * w.N >= (int64_t{16} << 20)));
+  return PickStreamShape(w, M, 0, 0).segs > 0 &&
+         (M <= 32 || w.K * w.N >= (int64_t{16} << 20) || StreamEven(w));
 }
 
 size_t StreamPartialBytes(const WeightView &w, int64_t M, int segs) {
@@ -1757,7 +1767,7 @@ hipError_t LaunchStream(const WeightView &w, int64_t M, const float *A, float *Y
   int *exps = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *P = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
                                        RowExpBytes(w, M));
-  const bool cvt = StreamConverts(w, M, sh, gamma != nullptr);
+  const bool cvt = gamma == nullptr && StreamConverts(w, M, sh);
   StreamIn in{Ah, cvt ? A : nullptr, exps, nullptr, eps};
   hipError_t e = hipSuccess;
   if (!cvt) {

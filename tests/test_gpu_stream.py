@@ -294,3 +294,44 @@ def test_stream_largest_magnitudes(pkg, orc, cuda, K, N, bs, zp, M):
     assert np.isfinite(Yn).all()
     for m in (1, 2, M - 1):
         assert not Yn[m].any(), m
+
+
+def _graph_us(torch, call):
+    """GPU time of a call in us: the least of 10 replays of a graph of 50."""
+    call()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(50):
+            call()
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    best = float("inf")
+    for _ in range(10):
+        start.record()
+        g.replay()
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) * 20)
+    return best
+
+
+@pytest.mark.parametrize("K,N,M,segs,spw", [
+    (2048, 512, 17, 4, 4),   # one segment of 8 x 8 took 30% longer
+    (2048, 2048, 32, 4, 4),
+    (5120, 5120, 48, 5, 8),  # two column groups, four segments of 5 x 8: 25%
+])
+def test_stream_default_shape_is_not_slower(pkg, cuda, K, N, M, segs, spw):
+    """The default launch shape against a given one on the same weights: at
+    most 15% more time."""
+    import torch
+    B, S, Z = _weights(pkg, K, N, 128, True, K + N)
+    op = pkg.MatMulNBits(K, N, 4, 128).prepare(B, S, Z)
+    A = torch.from_numpy(pkg.workloads.make_activations(M, K, 1.0, M)).to(cuda)
+    out = torch.empty(M, N, device=cuda)
+    print(f"case stream shape time K={K} N={N} M={M} kernel={op.kernel_name(M)}", flush=True)
+    assert op.kernel_name(M) == "StreamKernel"
+    given = _graph_us(torch, lambda: op.run_kernel(A, pkg.KERNEL_STREAM, segs, spw, out=out))
+    auto = _graph_us(torch, lambda: op(A, out=out))
+    op.release()
+    print(f"  default {auto:.2f} us, {segs} segments of {spw} steps {given:.2f} us")
+    assert auto <= 1.15 * given
