@@ -223,10 +223,12 @@ int mnb_run_rmsnorm(const mnb_plan *plan, int64_t M, const float *dX, const floa
  * address is looked up on the first call on each device). No counterpart in
  * the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). Fails with MNB_ERR_WORKSPACE, before any launch, when the
- * workspace of the kernels mnb_run would launch for these M rows (at most
- * mnb_workspace_bytes(plan, M); e.g. the prefill GEMM above M * K * 2 of
- * about 32 MiB, or a gate/up plan's M x 2N scratch sum) exceeds the array. Every
+ * hipMalloc). Where the array does not hold the workspace of the kernel that
+ * mnb_run would take, another kernel of the same path that fits serves (17 to
+ * 64 rows whose K-split partial sums are large: the tiled GEMMs; the exact GEMM:
+ * launches of fewer rows, then the decode or generic kernels). Fails with
+ * MNB_ERR_WORKSPACE, before any launch, when none fits (e.g. the prefill GEMM
+ * above M * K * 2 of about 32 MiB, or a gate/up plan's M x 2N scratch sum). Every
  * call on a GPU shares that GPU's array: calls that overlap in time on one
  * GPU (several streams or threads) race and must be ordered by the caller.
  * No kernel reads scratch bytes it did not write in the same call, so the

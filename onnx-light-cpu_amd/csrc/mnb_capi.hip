@@ -830,15 +830,19 @@ static size_t ExactFitBytes(const mnb_plan *plan, int64_t M, int path) {
                    : GateUpScratchBytes(plan, rows) + mnb::ExactWorkspaceBytes(plan->view, rows);
 }
 
-// Workspace the automatic path (mnb_run) takes for M rows of dA: the chosen
-// kernel's own, plus a gate/up plan's scratch sum where its epilogue does not
-// apply the activation (the exact route: per group of 16 rows).
+// Workspace the automatic path takes for M rows of dA when kScratchBytes are to
+// be had: the chosen kernel's own, plus a gate/up plan's scratch sum where its
+// epilogue does not apply the activation (the exact route: per group of 16 rows).
 static size_t AutoWorkspaceBytes(const mnb_plan *plan, int64_t M, const float *dA) {
   const int path = SelectPath(plan, M, dA);
   switch (path) {
   case 1:
     return DecodeNeed(plan, M) + (GateUpFusedInGemv(plan, M, 1) ? 0 : GateUpScratchBytes(plan, M));
-  case 2: return mnb::GemmWorkspaceBytes(plan->view, M) + GateUpScratchBytes(plan, M);
+  case 2: {
+    const size_t scratch = GateUpScratchBytes(plan, M);
+    return mnb::GemmWorkspaceBytes(plan->view, M, kScratchBytes - std::min(scratch, kScratchBytes)) +
+           scratch;
+  }
   case 4: {
     const int64_t md = std::min<int64_t>(M, kExactGroupRows);
     return std::max(DecodeNeed(plan, md) + GateUpScratchBytes(plan, md),
@@ -880,10 +884,12 @@ static int RunExact(const mnb_plan *plan, int64_t rows, const float *dA, const f
 
 // One run of the plan. With gamma, dA is the un-normalized input of a fused
 // RMSNorm: only the M = 1 GEMV and the GEMM take it (each reduces the rows
-// itself); mnb_run_rmsnorm normalizes the input for the rest.
+// itself); mnb_run_rmsnorm normalizes the input for the rest. limit: the most
+// workspace a kernel of the GEMM path may be chosen for (the others of the path
+// take less); a caller's own workspace holds that of every choice.
 static int RunImpl(const mnb_plan *plan, int64_t M, const float *dA, const float *dBias, float *dY,
                    void *dWorkspace, size_t workspace_bytes, void *stream, int path,
-                   const float *gamma, float eps) {
+                   const float *gamma, float eps, size_t limit = SIZE_MAX) {
   if (plan == nullptr) return MNB_ERR_NULL_POINTER;
   if (M < 0 || M > (int64_t{1} << 30)) return MNB_ERR_BAD_SHAPE;
   if (M == 0) return MNB_OK;
@@ -934,8 +940,9 @@ static int RunImpl(const mnb_plan *plan, int64_t M, const float *dA, const float
   void *work = scratch > 0 ? static_cast<void *>(static_cast<char *>(dWorkspace) + scratch)
                            : dWorkspace;
   const size_t work_bytes = scratch > 0 ? workspace_bytes - scratch : workspace_bytes;
+  limit -= std::min(scratch, limit);
   if (path == 2 || path == 5) {
-    const size_t need = mnb::GemmWorkspaceBytes(plan->view, M);
+    const size_t need = mnb::GemmWorkspaceBytes(plan->view, M, limit);
     if (work == nullptr || work_bytes < need || (reinterpret_cast<uintptr_t>(work) % 16) != 0)
       return MNB_ERR_WORKSPACE;
   }
@@ -1008,7 +1015,7 @@ static int RunImpl(const mnb_plan *plan, int64_t M, const float *dA, const float
     fused = H != nullptr && M * plan->view.N * 2 < (int64_t{1} << 31) &&
             plan->view.N < (int64_t{1} << 22);
     e = mnb::LaunchGemm(plan->view, M, dA, Ys, work, s, fused ? H : nullptr, gamma, eps, dBias,
-                        &bias_done);
+                        &bias_done, limit);
     break;
   case 5:
     fused = H != nullptr && M * plan->view.N * 2 < (int64_t{1} << 31) &&
@@ -1261,7 +1268,8 @@ int mnb_run_no_alloc(const mnb_plan *plan, int64_t M, const float *dA, float *dY
   void *work = nullptr;
   st = ScratchAddress(cur, &work);
   if (st != MNB_OK) return st;
-  return mnb_run_ex(plan, M, dA, nullptr, dY, need > 0 ? work : nullptr, need, stream, 0);
+  return RunImpl(plan, M, dA, nullptr, dY, need > 0 ? work : nullptr, need, stream, 0, nullptr, 0.0f,
+                 kScratchBytes);
 }
 
 } // extern "C"

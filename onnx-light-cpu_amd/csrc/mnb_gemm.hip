@@ -669,11 +669,13 @@ inline size_t AImageBytes(const WeightView &w, int64_t M) {
   return static_cast<size_t>(PaddedRows(M)) * static_cast<size_t>(w.K) * 2;
 }
 
-inline size_t RowExpBytes(const WeightView &w, int64_t M) {
-  // StreamKernel (at most 64 rows): an exponent and a sum of squares per row
-  // and chunk of K
-  const size_t chunks = M <= 64 ? static_cast<size_t>((w.K + kChunkK - 1) / kChunkK) : 1;
-  return (static_cast<size_t>(PaddedRows(M)) * 4 * chunks + 255) / 256 * 256;
+inline size_t RowExpBytes(int64_t M) {
+  return (static_cast<size_t>(PaddedRows(M)) * 4 + 255) / 256 * 256;
+}
+// StreamKernel (at most 64 rows): an exponent and a sum of squares per row and
+// chunk of K.
+inline size_t StreamExpBytes(const WeightView &w, int64_t M) {
+  return RowExpBytes(M) * static_cast<size_t>((w.K + kChunkK - 1) / kChunkK);
 }
 
 inline size_t PartialBytes(const WeightView &w, int64_t M, const Shape &sh) {
@@ -716,7 +718,7 @@ hipError_t LaunchBM(const WeightView &w, int64_t M, const float *A, float *Y, vo
   uint4 *Ah = static_cast<uint4 *>(work);
   int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *partials = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                              RowExpBytes(w, M));
+                                              RowExpBytes(M));
   hipError_t e = gamma != nullptr
                      ? LaunchConvertA<BM, true>(w, M, A, Ah, row_exp, s, gamma, eps)
                      : LaunchConvertA<BM, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
@@ -1621,18 +1623,13 @@ bool PrefillSupportsM(const WeightView &w, int64_t M) {
          (M + kPTM - 1) / kPTM * ((w.N + kPTN - 1) / kPTN) * kMaxSplits < (int64_t{1} << 31);
 }
 
-// Weights that the prefill kernel keeps above 32 rows: K / 32 steps that
-// segments of 8 x 16 steps do not divide, cut evenly into so many segments
-// (of 4 or 8 wavefronts of 4, 8 or 16 steps, covering 85% of the CUs) that
-// groups x segments are more than three per CU. Streaming them was slower than
-// the prefill kernel before the activations came in operand order; now it is
-// 8 to 16% faster (K = 5120, N = 13824 at M = 33 / 64 26.7 / 29.3 against
-// 29.0 / 32.3 us, K = 3584, N = 18944 23.7 / 27.2 against 28.2 / 31.4), but
-// their route is part of what the tests fix, so it stays.
-bool StreamCrowded(const WeightView &w, int64_t M) {
+// Weights whose K / 32 steps, cut evenly into segments (of 4 or 8 wavefronts of
+// 4, 8 or 16 steps, covering 85% of the CUs), make more than three groups x
+// segments per CU.
+bool StreamManyGroups(const WeightView &w, int64_t M) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
   const int T = static_cast<int>(w.K / 32);
-  if (M <= 32 || T % 128 == 0) return false;
+  if (M <= 32) return false;
   int best = 0;
   for (int segs = 1; segs <= kMaxSplits; ++segs) {
     const int per = T % segs == 0 ? T / segs : 0;
@@ -1642,6 +1639,16 @@ bool StreamCrowded(const WeightView &w, int64_t M) {
   }
   return (best > 1 || (best == 1 && M > 48)) &&
          groups * best > 3 * static_cast<int64_t>(w.num_cus);
+}
+
+// Those of them that the prefill kernel keeps above 32 rows: K / 32 steps that
+// segments of 8 x 16 steps do not divide. Streaming them was slower than
+// the prefill kernel before the activations came in operand order; now it is
+// 8 to 16% faster (K = 5120, N = 13824 at M = 33 / 64 26.7 / 29.3 against
+// 29.0 / 32.3 us, K = 3584, N = 18944 23.7 / 27.2 against 28.2 / 31.4), but
+// their route is part of what the tests fix, so it stays.
+bool StreamCrowded(const WeightView &w, int64_t M) {
+  return (w.K / 32) % 128 != 0 && StreamManyGroups(w, M);
 }
 
 // The prefill kernel serves the automatic GEMM path
@@ -1659,18 +1666,17 @@ bool StreamCrowded(const WeightView &w, int64_t M) {
 // 77.2, o and c4 within 3%; M = 256 gate+up 84.8 -> 63.8, qkv 34.6 -> about
 // 32, down 56.8 -> 50.0; with fewer than 12 k-tiles per split (o and c4 at
 // M <= 256, qkv at M = 128) GemmKernel's smaller tiles were 1-2 us faster;
-// - from 33 rows where the streaming kernel's launch is crowded (above).
-bool StreamSupportsM(const WeightView &w, int64_t M);
-
+// - from 33 rows where groups x segments are many (above).
+// Asked where the streaming kernel does not serve: its rows, sizes or routes, or
+// too little workspace.
 bool UsePrefill(const WeightView &w, int64_t M) {
   if (!PrefillSupportsM(w, M)) return false;
   // 17-64 rows the streaming kernel does not serve, on weights of 192 Mi
   // elements and more: the prefill kernel's tiles over GemmKernel's (K =
   // 29568, N = 8192 at M = 17 / 32 / 64: 66.5 / 67.2 / 74.1 against 80.2 /
   // 81.6 / 92.3 us; smaller weights stay: K = 20608, N = 2048 45 against 27).
-  const bool large_unstreamed = M >= 17 && !StreamSupportsM(w, M) &&
-                                w.K * w.N >= (int64_t{192} << 20);
-  if (M < 65 && !StreamCrowded(w, M) && !large_unstreamed) return false;
+  const bool large = M >= 17 && w.K * w.N >= (int64_t{192} << 20);
+  if (M < 65 && !large && !StreamManyGroups(w, M)) return false;
   const int64_t tiles = (M + kPTM - 1) / kPTM * ((w.N + kPTN - 1) / kPTN);
   const int64_t cus = w.num_cus;
   if (tiles < cus) {
@@ -1731,19 +1737,30 @@ size_t StreamPartialBytes(const WeightView &w, int64_t M, int segs) {
 
 } // namespace
 
-size_t GemmWorkspaceBytes(const WeightView &w, int64_t M) {
+// Without StreamKernel.
+static size_t TiledWorkspaceBytes(const WeightView &w, int64_t M) {
   size_t partial = w.B != nullptr ? PartialBytes(w, M, PickShape(w, M)) : 0;
   if (PrefillSupportsM(w, M)) partial = std::max(partial, PrefillPartialBytes(w, M));
-  if (StreamSupportsM(w, M))
-    partial = std::max(partial, StreamPartialBytes(w, M, PickStreamShape(w, M, 0, 0).segs));
-  return AImageBytes(w, M) + RowExpBytes(w, M) + partial;
+  return AImageBytes(w, M) + RowExpBytes(M) + partial;
+}
+
+// Its partial sums can be far larger than the tiled kernels' (K = 8320, N =
+// 11008 at M = 64 36 MB against 13): with less to be had those serve.
+static bool GemmStreams(const WeightView &w, int64_t M, size_t limit) {
+  return StreamSupportsM(w, M) &&
+         std::max(StreamWorkspaceBytes(w, M, 0, 0), TiledWorkspaceBytes(w, M)) <= limit;
+}
+
+size_t GemmWorkspaceBytes(const WeightView &w, int64_t M, size_t limit) {
+  const size_t tiled = TiledWorkspaceBytes(w, M);
+  return GemmStreams(w, M, limit) ? std::max(tiled, StreamWorkspaceBytes(w, M, 0, 0)) : tiled;
 }
 
 bool StreamSupports(const WeightView &w, int64_t M) { return StreamSupportsM(w, M); }
 
 size_t StreamWorkspaceBytes(const WeightView &w, int64_t M, int segs, int spw) {
   const StreamShape sh = PickStreamShape(w, M, segs, spw);
-  return AImageBytes(w, M) + RowExpBytes(w, M) + StreamPartialBytes(w, M, sh.segs);
+  return AImageBytes(w, M) + StreamExpBytes(w, M) + StreamPartialBytes(w, M, sh.segs);
 }
 
 // The epilogue finishes fragments wave, wave + wpg, ... up to TG of them per
@@ -1766,7 +1783,7 @@ hipError_t LaunchStream(const WeightView &w, int64_t M, const float *A, float *Y
   uint4 *Ah = static_cast<uint4 *>(work);
   int *exps = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *P = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                       RowExpBytes(w, M));
+                                       StreamExpBytes(w, M));
   const bool cvt = gamma == nullptr && StreamConverts(w, M, sh);
   StreamIn in{Ah, cvt ? A : nullptr, exps, nullptr, eps};
   hipError_t e = hipSuccess;
@@ -1833,7 +1850,7 @@ static hipError_t LaunchPrefillGemm(const WeightView &w, int64_t M, const float 
   uint4 *Ah = static_cast<uint4 *>(work);
   int *row_exp = reinterpret_cast<int *>(static_cast<char *>(work) + AImageBytes(w, M));
   float *partials = reinterpret_cast<float *>(static_cast<char *>(work) + AImageBytes(w, M) +
-                                              RowExpBytes(w, M));
+                                              RowExpBytes(M));
   hipError_t e = gamma != nullptr
                      ? LaunchConvertA<kPTM, true>(w, M, A, Ah, row_exp, s, gamma, eps)
                      : LaunchConvertA<kPTM, false>(w, M, A, Ah, row_exp, s, nullptr, 0.0f);
@@ -1869,7 +1886,7 @@ static hipError_t LaunchWideGemm(const WeightView &w, int64_t M, const float *A,
 }
 
 size_t GemmShapeWorkspaceBytes(const WeightView &w, int64_t M, int splits) {
-  return AImageBytes(w, M) + RowExpBytes(w, M) + PartialBytes(w, M, MakeShape(w, 32, splits));
+  return AImageBytes(w, M) + RowExpBytes(M) + PartialBytes(w, M, MakeShape(w, 32, splits));
 }
 
 bool GemmSupports(const WeightView &w, int64_t M) {
@@ -1918,9 +1935,9 @@ hipError_t LaunchGemmShape(const WeightView &w, int64_t M, const float *A, float
 
 hipError_t LaunchGemm(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                       hipStream_t s, float *H, const float *gamma, float eps, const float *bias,
-                      bool *bias_done) {
+                      bool *bias_done, size_t limit) {
   if (bias_done != nullptr) *bias_done = false;
-  if (StreamSupportsM(w, M)) {
+  if (GemmStreams(w, M, limit)) {
     if (bias_done != nullptr) *bias_done = bias != nullptr;
     return LaunchStream(w, M, A, Y, work, s, H, gamma, eps, bias, 0, 0);
   }

@@ -251,9 +251,12 @@ hipError_t LaunchSumPartials(float *Y, const float *P, int64_t mn, int parts, fl
 // where their tiles fill the CUs; all three add `bias` (N floats) themselves
 // and then set *bias_done.
 // Otherwise GemmKernel (BM x 128 tiles over the original layout) serves.
+// limit: where StreamKernel's workspace would exceed it, the others serve its
+// rows (GemmWorkspaceBytes with the same limit).
 hipError_t LaunchGemm(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                       hipStream_t s, float *H = nullptr, const float *gamma = nullptr,
-                      float eps = 0.0f, const float *bias = nullptr, bool *bias_done = nullptr);
+                      float eps = 0.0f, const float *bias = nullptr, bool *bias_done = nullptr,
+                      size_t limit = SIZE_MAX);
 bool GemmUsesPrefill(const WeightView &w, int64_t M);
 bool GemmUsesStream(const WeightView &w, int64_t M);
 bool GemmUsesWide(const WeightView &w, int64_t M);
@@ -295,7 +298,7 @@ hipError_t LaunchPrefillRelayout(const WeightView &w, uint8_t *Bp, uint8_t *Sp, 
 bool GemmSupports(const WeightView &w, int64_t M);
 // GemmKernel itself (the original layout).
 bool GemmKernelSupports(const WeightView &w, int64_t M);
-size_t GemmWorkspaceBytes(const WeightView &w, int64_t M);
+size_t GemmWorkspaceBytes(const WeightView &w, int64_t M, size_t limit = SIZE_MAX);
 // Same with an explicit tile height (32, 64 or 128; 0 picks both;
 // kPrefillTileCode = the prefill kernel) and split count (1..16), for
 // tuning; `work` then holds GemmShapeWorkspaceBytes(w, M, splits) bytes.

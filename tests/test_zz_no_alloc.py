@@ -99,3 +99,26 @@ def test_no_alloc_rejects_sizes_beyond_the_scratch(pkg, cuda):
     print(f"case no-alloc M={M2} workspace={op.workspace_bytes(M2)}", flush=True)
     np.testing.assert_array_equal(_no_alloc(pkg, op, A2, N), op(A2).cpu().numpy())
     op.release()
+
+
+@pytest.mark.parametrize("K,N,Ms", [
+    (15488, 8192, (64, 17)),  # 64 rows: the streaming kernel's partial sums exceed the scratch
+    (11392, 11008, (64, 49)),
+])
+def test_no_alloc_takes_a_kernel_that_fits_the_scratch(pkg, orc, cuda, K, N, Ms):
+    """Where mnb_run's kernel needs more workspace than the scratch holds but
+    another kernel of the path does not, the call takes that one."""
+    import torch
+    p = pkg.workloads.Projection("fit", K, N, 128, True)
+    B, S, Z = pkg.workloads.make_weights(p, 77)
+    op = pkg.MatMulNBits(K, N, 4, 128).prepare(B, S, Z)
+    cols = np.unique(np.concatenate([np.random.default_rng(K).integers(0, N, 60), [0, N - 1]]))
+    assert op.workspace_bytes(Ms[0]) > 32 << 20
+    for M in Ms:
+        A = pkg.workloads.make_activations(M, K, 1.0, 78 + M)
+        print(f"case no-alloc fit K={K} N={N} M={M} workspace={op.workspace_bytes(M)}", flush=True)
+        Y = _no_alloc(pkg, op, torch.from_numpy(A).to(cuda), N)
+        y64 = orc.matmul_nbits_f64(A, B[cols], S[cols], Z[cols], K, len(cols), 128)
+        assert orc.l2_rel_error(Y[:, cols], y64) <= GEMM_TOL
+        assert np.isfinite(Y).all()
+    op.release()
