@@ -132,9 +132,9 @@ __global__ __launch_bounds__(64) void SplitActKernel(const float *__restrict__ A
   for (int c = 0; c < 4; ++c) amax = fmaxf(amax, fmaxf(fabsf(v0[c]), fabsf(v1[c])));
   amax = HalfMax(amax);
   // The largest magnitude times 2^e in [2^14, 2^15); ldexp is exact for
-  // every e this gives (|e| <= 163), subnormal inputs included. A zero, inf
-  // or NaN maximum gives e = 0 (inf and NaN then propagate).
-  const int e = RangeExponent(amax, 14);
+  // every e this gives (|e| <= 163), subnormal inputs included; inf and NaN
+  // propagate in their first term.
+  const int e = SplitExponent(amax, 14);
   if (ch == 0) exps[u * kTok + t] = e;
   half8 h[kTerms];
 #pragma unroll
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void DecodeFragKernel(
             amax = fmaxf(amax, fmaxf(fabsf(raw[k][0][v]), fabsf(raw[k][1][v])));
         amax = fmaxf(amax, Xor16(amax));
         amax = fmaxf(amax, __shfl_xor(amax, 32));
-        se = RangeExponent(amax, 14);
+        se = SplitExponent(amax, 14);
         int ev[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int v = 0; v < kTPL; ++v) ev[v] = __shfl(se, (16 / TOKS) * (kTPL * qd + v));

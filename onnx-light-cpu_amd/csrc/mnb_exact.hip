@@ -123,9 +123,9 @@ __global__ __launch_bounds__(512) void SplitRowsKernel(const float *__restrict__
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < 8; ++w) amax = fmaxf(amax, red[w][r]);
-  // exact for every e this gives, subnormal inputs included; a zero, inf or
-  // NaN maximum gives e = 0 (inf and NaN then propagate)
-  const int e = RangeExponent(amax, kRowExpTarget);
+  // exact for every e this gives, subnormal inputs included; inf and NaN
+  // propagate in their first term
+  const int e = SplitExponent(amax, kRowExpTarget);
   if (threadIdx.x < 16) exps[static_cast<size_t>(u) * rows_padded + 16 * mt + lane] = e;
   half8 h[TERMS];
 #pragma unroll

@@ -265,12 +265,7 @@ __global__ __launch_bounds__(64 * kWaves) void GemvMfmaKernel(
     amax = RowMax16(amax);
     // e puts the largest magnitude in [2^14, 2^15); applied with ldexp, which
     // is exact for every e this gives (|e| <= 163), subnormal inputs included.
-    int e = 0;
-    if (amax > 0.f && __builtin_isfinite(amax)) {
-      int ex;
-      frexpf(amax, &ex);  // amax < 2^ex
-      e = 15 - ex;
-    }
+    const int e = SplitExponent(amax, 14);
     if (ac == 0) reinterpret_cast<int *>(lds_e)[at] = e;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {  // k-unit 4 c + u of the range (8 values)

@@ -81,6 +81,15 @@ __device__ __forceinline__ int RangeExponent(float amax, int target) {
   return target - (e - 1);
 }
 
+// The same for the kernels that split activations into fp16 terms, but an
+// infinite maximum counts as the largest finite value: unscaled, finite values
+// of 65520 and more beside the infinity would be infinite in fp16 too, and their
+// terms or signs make NaN where fp32 keeps the infinity. What the scaling loses
+// of them does not matter: the infinity decides every sum that it enters.
+__device__ __forceinline__ int SplitExponent(float amax, int target) {
+  return RangeExponent(fminf(amax, 3.402823466e38f), target);
+}
+
 // Exponent target of the plan's per-weight-row scale exponents: the largest
 // block scale of row n times 2^col_exp[n] lies in [2^11, 2^12), so every
 // block scale down to 2^-25 of it is a normal fp16 number and

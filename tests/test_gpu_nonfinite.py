@@ -136,3 +136,53 @@ def test_non_finite_rows_partial_unit(pkg, orc, cuda, K, M, bad):
     B, S, Z = W.make_weights(p, K + 2)
     A = W.make_activations(M, p.K, 1.0, K + 3 + M)
     _check_row(pkg, orc, cuda, p.K, p.N, p.block_size, B, S, Z, A, M, bad, f"K={K} N=512")
+
+
+def _plant_beside_large(A, row, bad):
+    """An infinity (or both) at k = 37 (and 90) of the row, beside finite values
+    that overflow fp16 unless they are scaled, of both signs."""
+    Ab = A.copy()
+    Ab[row, 5], Ab[row, 36], Ab[row, 38], Ab[row, 61] = 7e4, -1e6, 1e30, -3e34
+    Ab[row, 37] = -np.inf if bad == "-inf" else np.inf
+    if bad == "mixed":
+        Ab[row, 90] = -np.inf
+    return Ab
+
+
+@pytest.mark.parametrize("K,N,bs,zp,level,M", [
+    (4096, 1024, 128, True, 0, 4),    # the decode kernels on both layouts
+    (4096, 1024, 32, False, 0, 16),   # DecodeFragKernel's split in the kernel, 16 rows
+    (14336, 512, 128, True, 0, 8),    # SplitActKernel, 8 rows
+    (4096, 1026, 128, True, 0, 8),    # N % 4: the original layout's MFMA decode
+    (1024, 512, 64, True, 1, 32),     # ExactKernel, two terms
+    (1003, 70, 32, True, 0, 20),      # ExactKernel, three terms
+])
+@pytest.mark.parametrize("bad", ["+inf", "-inf", "mixed"])
+def test_infinity_beside_large_values(pkg, orc, cuda, K, N, bs, zp, level, M, bad):
+    """An infinite activation with finite ones of 7e4 to 3e34 in the same 32 k,
+    in the kernels that keep fp32 activations: the reference's kinds, which the
+    infinity alone decides (3e34 times any weight here is finite in fp32), and
+    every other row as without them. (The fp16 GEMMs convert a row that holds an
+    infinity unscaled, as the reference's conversion would.)"""
+    import torch
+    p = pkg.workloads.Projection("large", K, N, bs, zp)
+    B, S, Z = pkg.workloads.make_weights(p, K + N + 3)
+    A = pkg.workloads.make_activations(M, K, 1.0, K + M)
+    row = M // 2
+    Ab = _plant_beside_large(A, row, bad)
+    op = pkg.MatMulNBits(K, N, 4, bs, accuracy_level=level).prepare(B, S, Z)
+    print(f"case infinity beside large K={K} N={N} M={M} {bad}: {op.kernel_name(M)}", flush=True)
+    fp16 = {f"kernel {k}" for k in (pkg.KERNEL_GEMM, pkg.KERNEL_PREFILL, pkg.KERNEL_STREAM)}
+    runs = [r for r in _runs(pkg, op, A, Ab, cuda, M) if r[0] not in fp16]
+    op.release()
+    y32 = orc.matmul_nbits_ref_f32(Ab[row:row + 1], B, S, Z, K, N, bs)[0]
+    assert not np.isfinite(y32).any()
+    others = [m for m in range(M) if m != row]
+    failures = []
+    for name, y, yb in runs:
+        np.testing.assert_array_equal(yb[others], y[others], err_msg=name)
+        wrong = (_kinds(yb[row]) != _kinds(y32)).any(axis=0).sum()
+        if wrong:
+            failures.append(f"{name}: {wrong} of {N} outputs")
+    print("  checked " + ", ".join(r[0] for r in runs), flush=True)
+    assert not failures, failures
