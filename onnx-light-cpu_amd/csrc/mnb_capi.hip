@@ -216,8 +216,23 @@ int DerivePlanConstants(mnb_plan *p) {
     size_t zd_bytes = 0;
     const size_t bp_bytes = mnb::ExactRaggedLayoutBytes(p->view);
     const size_t sd_bytes = mnb::DecodeFragScaleBytes(p->view, &zd_bytes);
+    e = hipMalloc(reinterpret_cast<void **>(&p->dSd), sd_bytes);
+    if (e != hipSuccess) {
+      SetLastError("hipMalloc", e);
+      return MNB_ERR_ALLOC;
+    }
+    bool scales_ok = false;  // dSd holds at least 64 words
+    e = mnb::ExactRaggedScalesOk(p->view, reinterpret_cast<uint32_t *>(p->dSd), &scales_ok);
+    if (e != hipSuccess) {
+      SetLastError("plan constants", e);
+      return MNB_ERR_HIP;
+    }
+    if (!scales_ok) {  // GenericKernel serves the plan
+      (void)hipFree(p->dSd);
+      p->dSd = nullptr;
+      return MNB_OK;
+    }
     e = hipMalloc(reinterpret_cast<void **>(&p->dBp), bp_bytes);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&p->dSd), sd_bytes);
     if (e == hipSuccess && zd_bytes > 0) e = hipMalloc(reinterpret_cast<void **>(&p->dZd), zd_bytes);
     if (e != hipSuccess) {
       SetLastError("hipMalloc", e);

@@ -477,7 +477,34 @@ __global__ __launch_bounds__(256) void RelayoutRaggedKernel(const uint8_t *__res
                 : 0u;
 }
 
+// out[b]: the largest magnitude (its bits; infinite and NaN above all) of
+// workgroup b's share of the scales.
+__global__ __launch_bounds__(256) void LargestScaleKernel(const float *__restrict__ S, int64_t n,
+                                                          uint32_t *__restrict__ out) {
+  __shared__ uint32_t red[4];
+  uint32_t m = 0;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * 256)
+    m = max(m, __float_as_uint(S[i]) & 0x7FFFFFFFu);
+  for (int off = 32; off >= 1; off >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(m, off, 64)));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
 } // namespace ek
+
+hipError_t ExactRaggedScalesOk(const WeightView &w, uint32_t *work, bool *ok) {
+  uint32_t top[kScaleCheckWords];
+  hipLaunchKernelGGL(ek::LargestScaleKernel, dim3(kScaleCheckWords), dim3(256), 0, nullptr, w.scales,
+                     w.N * w.nb, work);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipMemcpy(top, work, sizeof(top), hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  constexpr uint32_t kLimit = (127u + 101u) << 23;  // 2^101
+  *ok = *std::max_element(top, top + kScaleCheckWords) < kLimit;
+  return hipSuccess;
+}
 
 bool ExactRaggedLayoutWanted(const WeightView &w) {
   return w.B != nullptr && ek::Ragged(w) && w.block_size >= 32 && w.K <= (int64_t{1} << 24) &&

@@ -244,6 +244,12 @@ hipError_t LaunchExact(const WeightView &w, int64_t M, const float *A, float *Y,
 // zero weights past the row's bytes (with Sd / Zd as for DecodeFragKernel).
 // No other kernel reads it: they take K % 64 == 0.
 bool ExactRaggedLayoutWanted(const WeightView &w);
+// Whether its sums stay in fp32's range with these scales: below 2^101, since a
+// unit's products reach 2^27 before its exponent is undone. (GenericKernel
+// multiplies dequantized weights, and an infinite scale would meet the zeros
+// past K.) Reads them on the null stream; `work` holds kScaleCheckWords words.
+constexpr int kScaleCheckWords = 64;
+hipError_t ExactRaggedScalesOk(const WeightView &w, uint32_t *work, bool *ok);
 size_t ExactRaggedLayoutBytes(const WeightView &w);
 hipError_t LaunchExactRaggedRelayout(const WeightView &w, uint8_t *Bp, hipStream_t s);
 // Y += P[0] + ... + P[parts - 1] over mn elements, in that order (then the

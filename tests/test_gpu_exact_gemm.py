@@ -145,3 +145,42 @@ def test_gate_up_and_graph(pkg, orc, cuda):
         h64 = orc.gate_up_silu_f64(A, *W[0], *W[1], K, I, bs)
         assert orc.normwise_max_error(out.cpu().numpy(), h64) <= 4 * TOL
     gu.release()
+
+
+@pytest.mark.parametrize("top,route", [
+    (1e32, "ExactKernel"),    # scales below 2^101: times the 2^27 of a unit's products finite
+    (1e36, "GenericKernel"),  # above: a unit's sum before its exponent is undone would overflow
+    (np.inf, "GenericKernel"),
+])
+def test_ragged_scales_at_the_end_of_the_range(pkg, orc, cuda, top, route):
+    """Weight scales near fp32's largest with activations near its smallest:
+    finite outputs stay finite, and an infinite scale gives its weight row the
+    reference's kinds (it meets no value past K)."""
+    import torch
+    K, N, bs, M = 1060, 70, 32, 20
+    p = pkg.workloads.Projection("scales", K, N, bs, True)
+    B, S, Z = pkg.workloads.make_weights(p, 21)
+    A = pkg.workloads.make_activations(M, K, 1.0, 22)
+    if np.isinf(top):
+        S[9, -1] = np.inf
+        B[9, -1], Z[9, -1] = 0x99, 0x33  # q - zp = 6 in the last block: A's sign decides
+        A[:, K // bs * bs:] = np.abs(A[:, K // bs * bs:]) + 0.5
+    else:
+        S[9] *= np.float32(top)
+        A *= np.float32(1e-30)
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare(B, S, Z)
+    name = op.kernel_name(M)
+    print(f"case exact scales {top} kernel={name}", flush=True)
+    Y = op(torch.from_numpy(A).to(cuda)).cpu().numpy()
+    op.release()
+    ref = orc.matmul_nbits_ref_f32(A, B, S, Z, K, N, bs)
+    if np.isinf(top):
+        assert np.isposinf(ref[:, 9]).all()
+        np.testing.assert_array_equal(np.isposinf(Y), np.isposinf(ref))
+        assert np.isfinite(np.delete(Y, 9, axis=1)).all()
+    else:
+        assert np.isfinite(ref).all() and np.isfinite(Y).all()
+        y64 = orc.matmul_nbits_f64(A, B, S, Z, K, N, bs)
+        for n in (9, 10):
+            assert orc.normwise_max_error(Y[:, n:n + 1], y64[:, n:n + 1]) <= TOL
+    assert name == route
