@@ -756,8 +756,9 @@ static bool Fp32ActivationsOnly(const mnb_plan *plan) { return plan->desc.accura
 // Rows of the first exact-GEMM launch for M rows of an automatic (or path 4)
 // run whose selected path is `path`, with work_bytes of workspace; 0 where the
 // other kernels of that path serve.
-// - 64-k plans (path 4): whole groups of 16 rows from 32 rows up, bit-identical
-//   to the decode kernels' groups, which serve the remaining rows.
+// - 64-k plans (path 4): whole groups of 16 rows, bit-identical to the decode
+//   kernels' groups, which serve the remaining rows: from 64 rows up, and 32 or
+//   48 where mnb::ExactBeatsGroups.
 // - K that 64-k tiles do not divide, all rows: path 4 (K a multiple of 32,
 //   above 16 rows), and path 3 where GenericKernel's one wavefront per column
 //   takes longer than this route's three launches: its time grows by about
@@ -783,6 +784,7 @@ static int64_t ExactRows(const mnb_plan *plan, int64_t M, int path, size_t work_
   if (path == 3 ? !ExactBeatsGeneric(plan, M) : M < (ragged ? 17 : 32)) return 0;
   int64_t rows = std::min(M, kExactMaxRows) / step * step;
   while (mnb::ExactSupports(plan->view, rows)) {
+    if (!ragged && rows < 64 && !mnb::ExactBeatsGroups(plan->view, rows)) break;
     if (GateUpScratchBytes(plan, rows) + mnb::ExactWorkspaceBytes(plan->view, rows) <= work_bytes)
       return rows;
     if (rows <= 32) break;

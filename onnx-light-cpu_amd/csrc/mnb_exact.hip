@@ -534,6 +534,28 @@ bool ExactSupports(const WeightView &w, int64_t M) {
          tiles * std::max(16, ek::Units(w)) < (int64_t{1} << 31);
 }
 
+// A workgroup multiplies a run of K one unit after the other (2.8 us each) while
+// DecodeFragKernel spreads it over wavefronts, so with few rows long runs are
+// the decode kernel's. Estimates in us; over 42 weights and two block sizes the
+// faster one is taken but for K = 8192, N = 28672 at 48 rows with 128-wide blocks
+// (92.9 by groups, 102.8 taken) and some within 4%. us, groups against this, at
+// 32 / 48 rows: K = 14336, N = 4096 (runs of 14) 32.4 /
+// 49.0 against 50.2 / 51.8; K = N = 4096 (4) 19.3 / 28.4, 23.2 / 23.5; K =
+// 4096, N = 28672 (16) 42.1 / 58.7, 56.2 / 55.6; K = 14336, N = 11008 (14, but
+// three rounds of decode workgroups) 66.7 / 96.4, 56.4 / 75.5; K = N = 2048 (1)
+// 18.1 / 27.1, 14.5 / 14.8.
+bool ExactBeatsGroups(const WeightView &w, int64_t M) {
+  int run = 1, range = 1;
+  DecodeFragRuns(w, &run, &range);
+  const int64_t cus = std::max(1, w.num_cus), runs = (ek::Units(w) + run - 1) / run;
+  const int64_t tiles = ek::PaddedRows(w, M) / 32 * ((w.N + ek::kCols - 1) / ek::kCols);
+  const double exact = 11.5 + 2.8 * run * std::max(1.0, static_cast<double>(tiles * runs) / cus);
+  const int64_t rounds = ((w.N + 63) / 64 * runs + cus - 1) / cus;
+  const double group = (runs > 1 ? 8.3 : 6.3) + 0.43 * static_cast<double>(rounds * run) +
+                       (range > 1 ? 1.0 : 0.0);
+  return exact < group * static_cast<double>(M / 16);
+}
+
 size_t ExactWorkspaceBytes(const WeightView &w, int64_t M) {
   const ek::Shape sh = ek::MakeShape(w, M);
   const size_t parts = sh.all_runs ? 0 : static_cast<size_t>(sh.runs - 1);

@@ -240,6 +240,9 @@ bool ExactSupports(const WeightView &w, int64_t M);
 size_t ExactWorkspaceBytes(const WeightView &w, int64_t M);
 hipError_t LaunchExact(const WeightView &w, int64_t M, const float *A, float *Y, void *work,
                        hipStream_t s, float *H = nullptr, const float *bias = nullptr);
+// Whether M = 32 or 48 rows of a 64-k plan take less time than in the decode
+// kernel's groups of 16.
+bool ExactBeatsGroups(const WeightView &w, int64_t M);
 // The ragged layout: Bp for K % 64 != 0, the records of whole 64-k tiles with
 // zero weights past the row's bytes (with Sd / Zd as for DecodeFragKernel).
 // No other kernel reads it: they take K % 64 == 0.

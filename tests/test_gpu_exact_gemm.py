@@ -184,3 +184,67 @@ def test_ragged_scales_at_the_end_of_the_range(pkg, orc, cuda, top, route):
         for n in (9, 10):
             assert orc.normwise_max_error(Y[:, n:n + 1], y64[:, n:n + 1]) <= TOL
     assert name == route
+
+
+def _graph_us(torch, call):
+    """GPU time of a call in us: the least of 10 replays of a graph of 20."""
+    call()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for _ in range(20):
+            call()
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    best = float("inf")
+    for _ in range(10):
+        start.record()
+        g.replay()
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) * 50)
+    return best
+
+
+@pytest.mark.parametrize("K,N,bs,M", [
+    (14336, 4096, 32, 32),  # the exact GEMM took 50% longer than two groups
+    (14336, 4096, 32, 47),
+    (4096, 28672, 128, 32),
+    (2048, 2048, 128, 32),  # the exact GEMM's
+])
+def test_level_1_few_rows_take_the_faster_route(pkg, cuda, K, N, bs, M):
+    """accuracy_level 1 at two or three groups of 16 rows: at most 15% more time
+    than the decode kernel's groups one after the other."""
+    import torch
+    op, *_ = _plan(pkg, K, N, bs, True, K + N, level=1)
+    A = torch.from_numpy(pkg.workloads.make_activations(M, K, 1.0, M)).to(cuda)
+    out = torch.empty(M, N, device=cuda)
+    print(f"case exact few rows K={K} N={N} M={M}: {op.kernel_name(M)}", flush=True)
+
+    def groups():
+        for m0 in range(0, M, 16):
+            op(A[m0:m0 + 16], out=out[m0:m0 + 16], path=pkg.PATH_GEMV)
+
+    auto = _graph_us(torch, lambda: op(A, out=out))
+    ref = _graph_us(torch, groups)
+    op.release()
+    print(f"  automatic {auto:.1f} us, groups {ref:.1f} us")
+    assert auto <= 1.15 * ref
+
+
+@pytest.mark.parametrize("K,N,bs,zp", [
+    (4096, 28676, 32, True),     # two column groups per decode workgroup, the last half empty
+    (14336, 16260, 128, False),
+    (2048, 65540, 64, True),
+    (4096, 4096, 128, True),     # activations split in the decode kernel
+])
+def test_level_1_rows_are_the_decode_kernels_on_wide_weights(pkg, cuda, K, N, bs, zp):
+    import torch
+    M = 64
+    op, *_ = _plan(pkg, K, N, bs, zp, K + M, level=1)
+    A = torch.from_numpy(pkg.workloads.make_activations(M, K, 1.0, M + 2)).to(cuda)
+    print(f"case exact wide K={K} N={N} bs={bs} kernel={op.kernel_name(M)}", flush=True)
+    assert op.kernel_name(M) == "ExactKernel"
+    Y = op(A)
+    for m0 in range(0, M, 16):
+        assert torch.equal(Y[m0:m0 + 16], op(A[m0:m0 + 16].contiguous(), path=pkg.PATH_GEMV)), m0
+    op.release()
