@@ -206,7 +206,8 @@ int mnb_run_ex(const mnb_plan *plan, int64_t M, const float *dA, const float *dB
  * and sums x^2 per 256-k unit, the main kernel scales each row's sums by
  * 1/rms); the GEMM path: a per-row 1/rms pass, then gamma and 1/rms folded
  * into the GEMM's conversion of A to fp16; every other kernel (the fp32-FMA
- * decode fallbacks): the normalized input is written to the workspace first. Works on gate/up plans too (H of the
+ * decode fallbacks, the exact GEMM, the generic kernel): the normalized input is
+ * written to the workspace first, and mnb_run's route multiplies it. Works on gate/up plans too (H of the
  * normalized input). The workspace is required:
  * mnb_rmsnorm_workspace_bytes. */
 int mnb_rmsnorm_workspace_bytes(const mnb_plan *plan, int64_t M, size_t *bytes);

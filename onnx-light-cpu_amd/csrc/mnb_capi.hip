@@ -1105,7 +1105,9 @@ int mnb_run_rmsnorm(const mnb_plan *plan, int64_t M, const float *dX, const floa
     SetLastError("kernel launch", e);
     return MNB_ERR_HIP;
   }
-  return RunImpl(plan, M, Xn, nullptr, dY, rest, rest_bytes, stream, path, nullptr, 0.0f);
+  // as mnb_run would: path 3 given by name is GenericKernel, without the exact
+  // GEMM that the automatic path 3 takes and the workspace is sized for
+  return RunImpl(plan, M, Xn, nullptr, dY, rest, rest_bytes, stream, 0, nullptr, 0.0f);
 }
 
 int mnb_run_path(const mnb_plan *plan, int64_t M, const float *dA, float *dY, void *dWorkspace,

@@ -248,3 +248,29 @@ def test_level_1_rows_are_the_decode_kernels_on_wide_weights(pkg, cuda, K, N, bs
     for m0 in range(0, M, 16):
         assert torch.equal(Y[m0:m0 + 16], op(A[m0:m0 + 16].contiguous(), path=pkg.PATH_GEMV)), m0
     op.release()
+
+
+@pytest.mark.parametrize("K,N,M", [
+    (2500, 500, 33),   # several K runs; two row tiles, the second of one row
+    (2500, 5000, 20),
+    (1004, 300, 17),   # the last unit and block filled in part
+])
+def test_rmsnorm_takes_the_exact_gemm(pkg, orc, cuda, K, N, M):
+    """mnb_run_rmsnorm on K % 64 != 0: the automatic route of the plain call,
+    which its workspace is sized for, on the normalized input."""
+    import torch
+    op, B, S, Z = _plan(pkg, K, N, 64, True, K + N + 5)
+    X = torch.from_numpy(pkg.workloads.make_activations(M, K, 3.0, M)).to(cuda)
+    gamma = np.random.default_rng(K).uniform(0.5, 1.5, K).astype(np.float32)
+    print(f"case exact rmsnorm K={K} N={N} M={M} kernel={op.kernel_name(M)}", flush=True)
+    assert op.kernel_name(M) == "ExactKernel"
+    Y = op.run_rmsnorm(X, torch.from_numpy(gamma).to(cuda), 1e-5)
+    # the normalized input as the call forms it, at the front of its workspace
+    Xn = op._work[:M * K * 4].view(torch.float32).view(M, K).clone()
+    plain = op(Xn)
+    op.release()
+    An = orc.rmsnorm_f64(X.cpu().numpy(), gamma, 1e-5)
+    assert orc.normwise_max_error(Xn.cpu().numpy(), An) <= 1e-6
+    assert torch.equal(Y, plain)
+    y64 = orc.matmul_nbits_f64(An.astype(np.float32), B, S, Z, K, N, 64)
+    assert orc.normwise_max_error(Y.cpu().numpy(), y64) <= 2 * TOL
