@@ -117,6 +117,7 @@ void FillView(mnb_plan *p) {
   p->view.block_size = p->desc.block_size;
   p->view.log2_bs = Log2(p->desc.block_size);
   p->view.num_cus = DeviceCUs(p->device);
+  mnb::SetStreamShapes(&p->view);
 }
 
 void FreePlanMemory(mnb_plan *p) {

@@ -1395,10 +1395,6 @@ __global__ __launch_bounds__(512) void StreamKernel(
   }
 }
 
-struct StreamShape {
-  int segs, wpg, spw;
-  int groups = 1;       // 64-row groups per workgroup
-};
 // Steps in flight with two groups per wavefront: 16 (w, sz) + 4 TG VGPRs each
 // beside 32 TG accumulators.
 template <int TG>
@@ -1432,14 +1428,9 @@ inline bool StreamConverts(const WeightView &w, int64_t M, const StreamShape &sh
 // K = 12288, N = 16384 at M = 17 six of 8 x 8 46.9, six of 4 x 16 35.4; K = 4096,
 // N = 28672 at M = 48 two groups, one of 8 x 16 26.3, one group 30.2.
 // M counts as the largest of its class: 24, 32, 48 or 64.
-inline StreamShape PickStreamShape(const WeightView &w, int64_t rows, int segs_req, int spw_req) {
+inline StreamShape SearchStreamShape(const WeightView &w, int64_t M) {
   const int64_t groups = (w.N + kSGroupRows - 1) / kSGroupRows;
   const int T = static_cast<int>(w.K / 32);
-  if (segs_req > 0 && spw_req > 0) {
-    const int per = segs_req * spw_req;
-    return StreamShape{segs_req, T % per == 0 ? T / per : 0, spw_req};
-  }
-  const int64_t M = rows <= 24 ? 24 : (rows + 15) / 16 * 16;
   const int tg = static_cast<int>((M + 15) / 16);
   StreamShape best{0, 0, 0};
   double best_us = 0.0;
@@ -1465,6 +1456,15 @@ inline StreamShape PickStreamShape(const WeightView &w, int64_t rows, int segs_r
       }
     }
   return best;
+}
+
+// The plan's shape for M rows (17 to 64), or the one asked for.
+inline StreamShape PickStreamShape(const WeightView &w, int64_t M, int segs_req, int spw_req) {
+  if (segs_req > 0 && spw_req > 0) {
+    const int per = segs_req * spw_req, T = static_cast<int>(w.K / 32);
+    return StreamShape{segs_req, T % per == 0 ? T / per : 0, spw_req};
+  }
+  return w.stream[M <= 24 ? 0 : M <= 32 ? 1 : M <= 48 ? 2 : 3];
 }
 
 // Whether K / 32 steps divide evenly into such segments.
@@ -1724,11 +1724,13 @@ size_t PrefillPartialBytes(const WeightView &w, int64_t M) {
 // against 16.3 / 16.9 us; N = 2048 14.6 / 16.4 against 18.2 / 19.3, N = 4096
 // 21.0 / 23.0 against 25.2 / 26.9; K = 2816, N = 20480 at M = 33 / 48 / 64
 // 23.0 / 24.8 / 28.9 against 26.8 / 27.9 / 28.9).
+bool StreamServes(const WeightView &w, int64_t M) {
+  if (!PrefillSupportsShape(w) || w.K > (int64_t{1} << 22) || StreamCrowded(w, M)) return false;
+  return M <= 32 || w.K * w.N >= (int64_t{16} << 20) || StreamEven(w);
+}
+
 bool StreamSupportsM(const WeightView &w, int64_t M) {
-  if (M < 17 || M > 64 || !PrefillSupportsShape(w) || w.K > (int64_t{1} << 22)) return false;
-  if (StreamCrowded(w, M)) return false;
-  return PickStreamShape(w, M, 0, 0).segs > 0 &&
-         (M <= 32 || w.K * w.N >= (int64_t{16} << 20) || StreamEven(w));
+  return M >= 17 && M <= 64 && PickStreamShape(w, M, 0, 0).segs > 0;
 }
 
 size_t StreamPartialBytes(const WeightView &w, int64_t M, int segs) {
@@ -1757,6 +1759,14 @@ size_t GemmWorkspaceBytes(const WeightView &w, int64_t M, size_t limit) {
 }
 
 bool StreamSupports(const WeightView &w, int64_t M) { return StreamSupportsM(w, M); }
+
+void SetStreamShapes(WeightView *w) {
+  // StreamServes and the search answer alike for all rows of a class.
+  constexpr int64_t kClassRows[4] = {24, 32, 48, 64};
+  for (int i = 0; i < 4; ++i)
+    w->stream[i] = StreamServes(*w, kClassRows[i]) ? SearchStreamShape(*w, kClassRows[i])
+                                                   : StreamShape{0, 0, 0};
+}
 
 size_t StreamWorkspaceBytes(const WeightView &w, int64_t M, int segs, int spw) {
   const StreamShape sh = PickStreamShape(w, M, segs, spw);

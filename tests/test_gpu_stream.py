@@ -335,3 +335,30 @@ def test_stream_default_shape_is_not_slower(pkg, cuda, K, N, M, segs, spw):
     op.release()
     print(f"  default {auto:.2f} us, {segs} segments of {spw} steps {given:.2f} us")
     assert auto <= 1.15 * given
+
+
+def test_workspace_query_host_time(pkg, cuda):
+    """A call of 17 to 64 rows asks for its launch shape several times. The
+    workspace query asks twice: against 8 rows, whose query has no shape to
+    find, it may take 0.2 us more (0.47 with a search each time, 0.01 without)."""
+    import ctypes
+    import time
+    B, S, Z = _weights(pkg, 4096, 4096, 128, True, 9)
+    op = pkg.MatMulNBits(4096, 4096, 4, 128).prepare(B, S, Z)
+    print(f"case stream workspace query {op.kernel_name(32)}", flush=True)
+    query, n = pkg.library().mnb_workspace_bytes, ctypes.c_size_t()
+    ref = ctypes.byref(n)
+
+    def us(M):
+        best = float("inf")
+        for _ in range(40):
+            t0 = time.perf_counter()
+            for _ in range(300):
+                query(op._plan, M, ref)
+            best = min(best, (time.perf_counter() - t0) / 300 * 1e6)
+        return best
+
+    extra = us(32) - us(8)
+    op.release()
+    print(f"  {extra:.2f} us more at 32 rows")
+    assert extra < 0.2
