@@ -142,8 +142,19 @@ void MatMulNBitsKernel::Run(RuntimeContext &rt) {
   Validate(*a, *b, *scales, zp, bias);
   TensorView &y = rt.MakeOutputTensor(0, DataType::kFloat, shape);
   const int64_t M = a->numel() / desc_.K;
-  const size_t need = WorkspaceBytes(*b, *scales, zp, M);
-  void *work = rt.Workspace(need);
+  size_t need = WorkspaceBytes(*b, *scales, zp, M);
+  void *work = nullptr;
+  try {
+    work = rt.Workspace(need);
+  } catch (const std::exception &) {
+    // On paths 3 and 4 most of it is the exact GEMM's; without that the generic
+    // kernel (no workspace) or the decode kernels on groups of 16 rows serve.
+    int path = 0;
+    CheckStatus(mnb_select_path(Plan(*b, *scales, zp), M, &path), "mnb_select_path");
+    if (path != 3 && path != 4) throw;
+    need = path == 3 ? 0 : WorkspaceBytes(*b, *scales, zp, 16);
+    work = rt.Workspace(need);
+  }
   (*this)(*a, *b, *scales, zp, y, rt.stream, work, need, bias);
 }
 

@@ -51,3 +51,35 @@ def test_node_matches_direct_call(pkg, orc, cuda, K, N, bs, zp, M):
     tol, metric = (2e-3, orc.l2_rel_error) if M > 16 else (1e-5, orc.normwise_max_error)
     assert metric(y_node.cpu().numpy(), y64) <= tol
     op.release()
+
+
+@pytest.mark.parametrize("K,N,M,level", [
+    (300, 200, 20, 0),     # K no multiple of 32: the exact GEMM, or GenericKernel without workspace
+    (2500, 501, 33, 0),
+    (1024, 2048, 256, 1),  # fp32 activations: the exact GEMM, or groups of 16 rows
+])
+def test_node_without_the_exact_gemms_workspace(pkg, cuda, K, N, M, level):
+    """Where the runtime's workspace holds what the kernels behind the exact
+    GEMM need (nothing for K that is no multiple of 32), but not the exact
+    GEMM's own, those kernels serve the node."""
+    import torch
+    bs = 32
+    B, S, Z = pkg.workloads.make_weights(pkg.workloads.Projection("t", K, N, bs, True), 23)
+    dA = torch.from_numpy(pkg.workloads.make_activations(M, K, 1.0, 24)).to(cuda)
+    dB, dS, dZ = (torch.from_numpy(x).to(cuda) for x in (B, S, Z))
+    op = pkg.MatMulNBits(K, N, 4, bs, level).prepare_device(dB, dS, dZ)
+    assert op.kernel_name(M) == "ExactKernel"
+    least = 0 if K % 32 else op.workspace_bytes(16)
+    assert least < op.workspace_bytes(M)
+    work = torch.empty(least, dtype=torch.uint8, device=cuda) if least else None
+    print(f"adapter least workspace K={K} N={N} M={M} level={level} {least} bytes of "
+          f"{op.workspace_bytes(M)}", flush=True)
+    pkg.register_kernels()
+    Y = torch.empty(M, N, device=cuda)
+    attrs = {"K": K, "N": N, "bits": 4, "block_size": bs, "accuracy_level": level}
+    pkg.run_node("com.microsoft", "MatMulNBits", attrs, _node_inputs(pkg, dA, dB, dS, dZ), Y,
+                 stream=torch.cuda.current_stream().cuda_stream, workspace=work)
+    want = op(dA, path=pkg.PATH_GENERIC) if K % 32 else op(dA)  # the exact GEMM has the groups' bits
+    torch.cuda.synchronize()
+    assert torch.equal(Y.cpu(), want.cpu())
+    op.release()
