@@ -255,7 +255,11 @@ class MatMulNBits:
         raw = _raw_stream(device) if stream is None else stream.cuda_stream
         if bias is not None and (bias.numel() != N or not bias.is_contiguous()):
             raise ValueError(f"{KERNEL_PREFIX}: bias must be a contiguous [N] tensor")
-        work = self.workspace(M, device, path)
+        if stream is None or K % 64 == 0:
+            work = self.workspace(M, device, path)
+        else:  # the run's own workspace: allocated on the stream that runs it
+            with torch.cuda.stream(torch.cuda.ExternalStream(raw, device)):
+                work = self.workspace(M, device, path)
         status = _lib.mnb_run_ex(self._plan, M, A2.data_ptr(),
                                  None if bias is None else bias.data_ptr(), out.data_ptr(),
                                  None if work is None else work.data_ptr(),
@@ -333,10 +337,16 @@ class MatMulNBits:
         return n.value
 
     def workspace(self, M: int, device, path: int = PATH_AUTO):
-        """Device workspace for M rows, kept and grown across calls (not during capture)."""
+        """Device workspace for M rows, kept and grown across calls (not during
+        capture). Where K is not a multiple of 64 each call has its own, in order
+        on the current stream: the generic kernel behind the exact GEMM takes
+        none, so that one object's calls may overlap on several streams."""
         need = self.workspace_bytes(M) if path != PATH_GENERIC else 0
         if need == 0:
             return None
+        if self.desc.K % 64 != 0:
+            import torch
+            return torch.empty(need, dtype=torch.uint8, device=device)
         if self._work is None or self._work.numel() < need or self._work.device != device:
             import torch
             self._work = torch.empty(need, dtype=torch.uint8, device=device)
