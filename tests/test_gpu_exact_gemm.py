@@ -121,8 +121,8 @@ def test_small_workspaces(pkg, orc, cuda, K, level):
 
 
 def test_gate_up_and_graph(pkg, orc, cuda):
-    """The gate/up activation behind one and several runs, and a captured call
-    replayed on changed activations."""
+    """The gate/up activation in the pass that adds the partial sums of two runs,
+    and a captured call replayed on changed activations."""
     import torch
     K, I, bs, M = 1000, 100, 32, 40
     p = pkg.workloads.Projection("gu", K, I, bs, True)
@@ -145,6 +145,34 @@ def test_gate_up_and_graph(pkg, orc, cuda):
         h64 = orc.gate_up_silu_f64(A, *W[0], *W[1], K, I, bs)
         assert orc.normwise_max_error(out.cpu().numpy(), h64) <= 4 * TOL
     gu.release()
+
+
+@pytest.mark.parametrize("K,I,bs,level,M", [
+    (200, 300, 64, 0, 37),     # one unit; 88 columns in the third tile, 5 rows in the second
+    (160, 33, 32, 0, 50),      # K an odd multiple of 32 (path 4), 66 columns
+    (1000, 1555, 128, 0, 1000),  # 416 tiles: one run of four units
+    (1024, 770, 64, 1, 2050),  # 448 tiles: every run in one workgroup; two rows by the decode kernels
+])
+def test_gate_up_in_the_epilogue(pkg, orc, cuda, K, I, bs, level, M):
+    """The gate/up activation in ExactKernel's own stores, where one workgroup
+    has all of K: half the columns, nothing written outside H."""
+    import torch
+    p = pkg.workloads.Projection("gu", K, I, bs, True)
+    W = [pkg.workloads.make_weights(p, s) for s in (71, 72)]
+    gu = pkg.GateUpSiLU(K, I, 4, bs, level).prepare(*W[0], *W[1])
+    print(f"case exact gate/up epilogue K={K} I={I} M={M} kernel={gu.kernel_name(M)}", flush=True)
+    assert gu.kernel_name(M) == "ExactKernel"
+    A = pkg.workloads.make_activations(M, K, 1.0, 73)
+    buf = torch.full((M * I + 8,), float("nan"), device=cuda)
+    out = buf[4:4 + M * I].view(M, I)
+    gu(torch.from_numpy(A).to(cuda), out=out)
+    H = out.cpu().numpy()
+    assert torch.isnan(buf[:4]).all() and torch.isnan(buf[4 + M * I:]).all()
+    gu.release()
+    assert np.isfinite(H).all()
+    rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 48)), [M - 2, M - 1]]))
+    h64 = orc.gate_up_silu_f64(A[rows], *W[0], *W[1], K, I, bs)
+    assert orc.normwise_max_error(H[rows], h64) <= 4 * TOL
 
 
 @pytest.mark.parametrize("top,route", [

@@ -206,11 +206,12 @@ def test_stream_shorter_last_segment_serves_up_to_32_rows(pkg, cuda):
 
 @pytest.mark.parametrize("K,N,bs,zp,M", [
     (512, 64, 32, True, 17),       # one group, one chunk of K, one row past a row tile
-    (1088, 132, 64, False, 33),    # 34 steps: a wavefront per 8 does not divide; ragged columns
+    (1152, 132, 64, False, 20),    # 36 steps, three segments of 4 x 4, the last shorter; ragged
+                                   # columns; a chunk that K does not fill
     (4096, 28672, 128, True, 48),  # two column groups per workgroup
     (4096, 28740, 32, False, 64),  # an odd group count: the last workgroup's second group is padding
-    (14336, 4096, 128, True, 64),  # seven wavefronts of 16 steps, four segments
-    (2624, 17408, 64, True, 40),   # two groups, a chunk that K does not fill
+    (14336, 4096, 128, True, 64),  # seven wavefronts of 16 steps, four segments, one group
+    (2816, 20480, 64, True, 64),   # two groups, a chunk that K does not fill
 ])
 def test_stream_shapes_rms_and_bias(pkg, orc, cuda, K, N, bs, zp, M):
     """The launch shapes of the streaming GEMM (wavefronts per workgroup, one
@@ -233,6 +234,7 @@ def test_stream_shapes_rms_and_bias(pkg, orc, cuda, K, N, bs, zp, M):
     bias = rng.standard_normal(N).astype(np.float32)
     gamma = rng.uniform(0.5, 1.5, K).astype(np.float32)
     print(f"case stream shapes K={K} N={N} bs={bs} M={M} kernel={op.kernel_name(M)}", flush=True)
+    assert op.kernel_name(M) == "StreamKernel"
     ref = lambda X: orc.matmul_nbits_f64(X, B[cols], S[cols], None if Z is None else Z[cols],
                                          K, len(cols), bs)
     y64 = ref(A)
@@ -247,20 +249,19 @@ def test_stream_shapes_rms_and_bias(pkg, orc, cuda, K, N, bs, zp, M):
     Yb = op(dA, bias=torch.from_numpy(bias).to(cuda)).cpu().numpy()
     np.testing.assert_array_equal(Yb, Y + bias[None, :])
     # rows whose squares stay in fp32's range
-    keep = [m for m in range(M) if m not in (1, 2)]
-    Yn = op.run_rmsnorm(dA[keep].contiguous(), torch.from_numpy(gamma).to(cuda), 1e-5).cpu().numpy()
-    n64 = ref(orc.rmsnorm_f64(A[keep].astype(np.float64), gamma.astype(np.float64), 1e-5).astype(np.float32))
-    for i in range(len(keep)):
-        if n64[i].any():
-            assert orc.l2_rel_error(Yn[i:i + 1, cols], n64[i:i + 1]) <= 2e-3, keep[i]
+    A[1:3] = pkg.workloads.make_activations(2, K, 1.0, M + 1)
+    Yn = op.run_rmsnorm(torch.from_numpy(A).to(cuda), torch.from_numpy(gamma).to(cuda),
+                        1e-5).cpu().numpy()
+    check(Yn, ref(orc.rmsnorm_f64(A.astype(np.float64), gamma.astype(np.float64),
+                                  1e-5).astype(np.float32)))
     op.release()
 
 
 @pytest.mark.parametrize("K,N,bs,zp,M", [
-    (4096, 4096, 128, False, 32),  # the wavefronts convert the activations; four segments
+    (4096, 4096, 128, False, 17),  # the wavefronts convert the activations; four segments
     (512, 64, 32, True, 40),       # the image, one group, one segment
     (4096, 28672, 128, True, 48),  # two column groups, one segment
-    (14336, 4096, 128, True, 64),  # two column groups, several segments
+    (14336, 4096, 128, True, 64),  # seven wavefronts, four segments
 ])
 def test_stream_largest_magnitudes(pkg, orc, cuda, K, N, bs, zp, M):
     """Rows near both ends of fp32: 1e36 times N(0, 1) gives outputs of up to
