@@ -7,7 +7,7 @@
 // per MFMA, which with the MFMAs' own issue fills 85% of a SIMD's cycles; here
 // it is 1.1 (132 -> 111 us at M = 512, K = 4096, N = 28672, one wave of
 // tiles; 1.24 PFLOP/s at M = 8192 against 1.09). What bounds it is the MFMAs
-// at the clock that their power leaves (62% of the cycles), and per tile the
+// at the clock that their power leaves (65% of the cycles), and per tile the
 // prologue and the 256 KiB of stores, which one workgroup per CU does not
 // overlap: a 32x32x16 form of the k-loop took as many cycles, and within 3%
 // as many without its LDS activation reads, half its copies or the
