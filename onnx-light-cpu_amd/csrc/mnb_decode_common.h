@@ -32,27 +32,12 @@ __device__ __forceinline__ float MixHi0(float a, uint32_t h) {
 }
 
 typedef _Float16 hf8 __attribute__((ext_vector_type(8)));
-typedef _Float16 hf2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
-  const hf2 r = __builtin_bit_cast(hf2, a) + __builtin_bit_cast(hf2, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
 
 // 8 nibbles (k order) of one word -> q - zp as fp16 in [0,4,1,5,2,6,3,7]
 // order, exact: (w & 0x000F000F) | 0x6400.. is the fp16 pair 1024 + q of
 // nibbles 0 | 4 (ulp 1 at 1024), (w & 0x00F000F0) | 0x5400.. the pair 64 + q
 // of nibbles 1 | 5 (ulp 1/16 at 64); the same of w >> 8 gives nibbles 2 | 6
 // and 3 | 7. neg_lo / neg_hi are the fp16 pairs -(1024 + zp) / -(64 + zp).
-// The masks sit in VGPRs (v_and_or_b32 takes no literal on gfx9).
-struct Masks {
-  uint32_t lo, hi, e1024, e64;
-};
-__device__ __forceinline__ Masks MakeMasks() {
-  Masks c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
-  return c;
-}
 __device__ __forceinline__ hf8 DecodeQ(uint32_t w, uint32_t neg_lo, uint32_t neg_hi,
                                          const Masks &c) {
   const uint32_t w8 = w >> 8;

@@ -75,12 +75,6 @@ constexpr int Stages() { return StageUnits<MI, TERMS>() * 16 * 4 <= 80 * 1024 ? 
 template <int MI, int TERMS>
 constexpr size_t LdsBytes() { return size_t{16} * StageUnits<MI, TERMS>() * Stages<MI, TERMS>(); }
 
-// s_waitcnt vmcnt(N), the other counters left free.
-template <int N>
-__device__ __forceinline__ void WaitVm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // One workgroup of 8 wavefronts per (256-k unit, group of 16 rows); wavefront
 // w takes step w, lane l the 8 values k = 256 u + 32 w + 8 (l >> 4) .. + 7 of
 // row l & 15. Rows of K floats need no alignment beyond 4 bytes.

@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256, 2) void GemmKernel(const uint4 *__restrict__ A
       r.zshift = 0;
     }
   };
-  const DequantConsts dq = MakeDequantConsts();
+  const Masks dq = MakeMasks();
   // The weight row's power-of-two exponent (plan time): its block scales times
   // 2^e_b are normal fp16 numbers and (q - zp) * scale stays below 65504.
   const int e_b = col_exp[min(n0 + b_row, N - 1)];
@@ -891,7 +891,7 @@ PrefillKernel(const uint4 *__restrict__ Ah, const uint8_t *__restrict__ Bp,
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const DequantConsts dq = MakeDequantConsts();
+  const Masks dq = MakeMasks();
   // Dequantized weight fragments of one 32-k step (MFMA A operands, slices j).
   auto dequant = [&](uint4 bw, uint4 sw, half8 (&bf)[4]) __attribute__((always_inline)) {
     const uint32_t w[4] = {bw.x, bw.y, bw.z, bw.w};
@@ -1284,7 +1284,7 @@ __global__ __launch_bounds__(512) void StreamKernel(
     }
   }
 
-  const DequantConsts dq = MakeDequantConsts();
+  const Masks dq = MakeMasks();
   floatx4 acc[G][TG][4];
 #pragma unroll
   for (int x = 0; x < G; ++x)

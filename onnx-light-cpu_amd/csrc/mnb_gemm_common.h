@@ -22,27 +22,9 @@ __device__ __forceinline__ uint32_t PackHalf2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
-__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
-  const half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
 __device__ __forceinline__ uint32_t PkMulF16(uint32_t a, uint32_t b) {
   const half2v r = __builtin_bit_cast(half2v, a) * __builtin_bit_cast(half2v, b);
   return __builtin_bit_cast(uint32_t, r);
-}
-
-// Per-thread constants of the dequantization, held in VGPRs (an empty asm
-// hides their values from the compiler): VOP3 instructions on gfx9 take no
-// literal, so with the masks as literals (w & m) | c costs two instructions
-// instead of one v_and_or_b32.
-struct DequantConsts {
-  uint32_t lo, hi, e1024, e64;  // 0x000F000F, 0x00F000F0, fp16 pairs 1024.0, 64.0
-};
-__device__ __forceinline__ DequantConsts MakeDequantConsts() {
-  DequantConsts c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
-  return c;
 }
 
 // Per (row, k-tile) operands of DequantWord: -(1024 + zp) and -(64 + zp)
@@ -65,7 +47,7 @@ __device__ __forceinline__ DequantRow MakeDequantRow(float s, uint32_t zp) {
 // and one multiply by the fp16 scale rounds the weight once. Per word: one
 // shift, four v_and_or_b32, four packed adds and four packed multiplies.
 __device__ __forceinline__ uint4 DequantWord(uint32_t w, const DequantRow &r,
-                                             const DequantConsts &c) {
+                                             const Masks &c) {
   const uint32_t w8 = w >> 8;
   const uint32_t h0 = (w & c.lo) | c.e1024;   // nibbles 0 | 4: 1024 + q
   const uint32_t h1 = (w & c.hi) | c.e64;     // nibbles 1 | 5: 64 + q
@@ -92,13 +74,6 @@ __device__ __forceinline__ DequantRow RowFromSz(uint32_t w) {
     r.neg_hi = 0xD480D480u;  // -(64 + 8)
   }
   return r;
-}
-
-// s_waitcnt vmcnt(N) with the other counters left free (gfx9 encoding: vmcnt
-// in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <int N>
-__device__ __forceinline__ void WaitVm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
 } // namespace gemm

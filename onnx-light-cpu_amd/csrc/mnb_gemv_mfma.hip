@@ -57,7 +57,6 @@ namespace mf {
 using namespace dec;
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -69,36 +68,6 @@ constexpr int kSteps = kKR / 32;                      // 32-k MFMA steps per ran
 constexpr int kStepUnits = 4 * kTok;                  // 16-byte A units per step and term
 constexpr int kTermUnits = kSteps * kStepUnits;       // 1024
 constexpr int kMaxSplits = 64;
-
-__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
-  const half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-struct Masks {
-  uint32_t lo, hi, e1024, e64;  // 0x000F000F, 0x00F000F0, fp16 pairs 1024.0, 64.0
-};
-__device__ __forceinline__ Masks MakeMasks() {
-  Masks c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
-  // Held in VGPRs: v_and_or_b32 (VOP3) takes no literal operand on gfx9.
-  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
-  return c;
-}
-
-// 8 nibbles (k order) of one word -> q - zp as fp16 in [0,4,1,5,2,6,3,7]
-// order, exact: (w & 0x000F000F) | 0x6400.. is the fp16 pair 1024 + q of
-// nibbles 0 | 4 (ulp 1 at 1024), (w & 0x00F000F0) | 0x5400.. the pair 64 + q
-// of nibbles 1 | 5 (ulp 1/16 at 64); the same of w >> 8 gives nibbles 2 | 6
-// and 3 | 7. neg_lo / neg_hi are the fp16 pairs -(1024 + zp) / -(64 + zp).
-__device__ __forceinline__ half8 DecodeQ(uint32_t w, uint32_t neg_lo, uint32_t neg_hi,
-                                         const Masks &c) {
-  const uint32_t w8 = w >> 8;
-  const uint4 r = make_uint4(PkAddF16((w & c.lo) | c.e1024, neg_lo),
-                             PkAddF16((w & c.hi) | c.e64, neg_hi),
-                             PkAddF16((w8 & c.lo) | c.e1024, neg_lo),
-                             PkAddF16((w8 & c.hi) | c.e64, neg_hi));
-  return __builtin_bit_cast(half8, r);
-}
 
 // Transposes the 4 x 4 dwords held by lanes c, c + 16, c + 32, c + 48 in
 // v[0..3] (lane group g, register j -> lane group j, register g): one

@@ -90,6 +90,33 @@ __device__ __forceinline__ int SplitExponent(float amax, int target) {
   return RangeExponent(fminf(amax, 3.402823466e38f), target);
 }
 
+// Two fp16 sums (one packed add).
+__device__ __forceinline__ uint32_t PkAddF16(uint32_t a, uint32_t b) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  const half2v r = __builtin_bit_cast(half2v, a) + __builtin_bit_cast(half2v, b);
+  return __builtin_bit_cast(uint32_t, r);
+}
+
+// Per-thread constants of the nibble decodes, held in VGPRs (an empty asm
+// hides their values from the compiler): VOP3 instructions on gfx9 take no
+// literal, so with the masks as literals (w & m) | c costs two instructions
+// instead of one v_and_or_b32.
+struct Masks {
+  uint32_t lo, hi, e1024, e64;  // 0x000F000F, 0x00F000F0, fp16 pairs 1024.0, 64.0
+};
+__device__ __forceinline__ Masks MakeMasks() {
+  Masks c{0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
+  __asm__ volatile("" : "+v"(c.lo), "+v"(c.hi), "+v"(c.e1024), "+v"(c.e64));
+  return c;
+}
+
+// s_waitcnt vmcnt(N) with the other counters left free (gfx9 encoding: vmcnt
+// in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
+template <int N>
+__device__ __forceinline__ void WaitVm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
 // Exponent target of the plan's per-weight-row scale exponents: the largest
 // block scale of row n times 2^col_exp[n] lies in [2^11, 2^12), so every
 // block scale down to 2^-25 of it is a normal fp16 number and

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     }(std::make_integer_sequence<int, kOps>{});
   };
 
-  const DequantConsts dq = MakeDequantConsts();
+  const Masks dq = MakeMasks();
   floatx4 acc[kMI][4];
 #pragma unroll
   for (int i = 0; i < kMI; ++i)
