@@ -458,17 +458,18 @@ __global__ __launch_bounds__(256) void RelayoutRaggedKernel(const uint8_t *__res
                                                             uint32_t *__restrict__ Bp, int64_t N,
                                                             int64_t row_bytes, int64_t T,
                                                             int64_t words) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= words) return;
-  const int j = static_cast<int>(idx & 3);
-  const int l = static_cast<int>((idx >> 2) & 63);
-  const int64_t gs = idx >> 8;
-  const int64_t s = gs % T, g = gs / T;
-  const int64_t n = 64 * g + 16 * j + (l & 15);
-  const int64_t byte = 16 * s + 4 * (l >> 4);
-  Bp[idx] = n < N && byte + 4 <= row_bytes
-                ? *reinterpret_cast<const uint32_t *>(B + n * row_bytes + byte)
-                : 0u;
+  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < words;
+       idx += static_cast<int64_t>(gridDim.x) * 256) {
+    const int j = static_cast<int>(idx & 3);
+    const int l = static_cast<int>((idx >> 2) & 63);
+    const int64_t gs = idx >> 8;
+    const int64_t s = gs % T, g = gs / T;
+    const int64_t n = 64 * g + 16 * j + (l & 15);
+    const int64_t byte = 16 * s + 4 * (l >> 4);
+    Bp[idx] = n < N && byte + 4 <= row_bytes
+                  ? *reinterpret_cast<const uint32_t *>(B + n * row_bytes + byte)
+                  : 0u;
+  }
 }
 
 // out[b]: the largest magnitude (its bits; infinite and NaN above all) of
@@ -511,9 +512,8 @@ size_t ExactRaggedLayoutBytes(const WeightView &w) {
 
 hipError_t LaunchExactRaggedRelayout(const WeightView &w, uint8_t *Bp, hipStream_t s) {
   const int64_t words = static_cast<int64_t>(ExactRaggedLayoutBytes(w) / 4);
-  hipLaunchKernelGGL(ek::RelayoutRaggedKernel, dim3(static_cast<unsigned>((words + 255) / 256)),
-                     dim3(256), 0, s, w.B, reinterpret_cast<uint32_t *>(Bp), w.N, w.row_bytes,
-                     ek::Steps(w), words);
+  hipLaunchKernelGGL(ek::RelayoutRaggedKernel, StrideGrid(words), dim3(256), 0, s, w.B,
+                     reinterpret_cast<uint32_t *>(Bp), w.N, w.row_bytes, ek::Steps(w), words);
   return hipGetLastError();
 }
 

@@ -117,6 +117,12 @@ __device__ __forceinline__ void WaitVm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
+// Workgroups of 256 threads for a kernel whose threads stride over n items: a
+// launch of 2^32 threads or more runs only their number modulo 2^32.
+inline dim3 StrideGrid(int64_t n) {
+  return dim3(static_cast<unsigned>(n < (int64_t{1} << 31) ? (n + 255) / 256 : 1 << 23));
+}
+
 // Exponent target of the plan's per-weight-row scale exponents: the largest
 // block scale of row n times 2^col_exp[n] lies in [2^11, 2^12), so every
 // block scale down to 2^-25 of it is a normal fp16 number and

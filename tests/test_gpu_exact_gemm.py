@@ -337,3 +337,30 @@ def test_ragged_calls_on_two_streams(pkg, cuda, explicit):
     op.release()
     for w, out in zip(want, outs):
         assert all(torch.equal(o.cpu(), w) for o in out)
+
+
+def test_ragged_weights_of_18_gb(pkg, orc, cuda):
+    """18 GB of weights: their re-laid copy has more than 2^32 words, and one
+    launch has fewer threads than that. Columns from its start, its end and both
+    sides of the word where the launch's threads would end."""
+    import torch
+    K, N, bs, M = 131073, 270000, 256, 2
+    nb = -(-K // bs)
+    if torch.cuda.mem_get_info(cuda)[0] < 40 << 30:
+        pytest.skip("less than 40 GiB of device memory free")
+    gen = torch.Generator(device=cuda).manual_seed(5)
+    B = torch.randint(0, 256, (N, nb, bs // 2), dtype=torch.uint8, device=cuda, generator=gen)
+    S = torch.rand((N, nb), device=cuda, generator=gen) * 0.015 + 0.005
+    A = pkg.workloads.make_activations(M, K, 1.0, 6)
+    print(f"case ragged 18 GB K={K} N={N} bs={bs} {B.numel()} bytes", flush=True)
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare_device(B, S)
+    assert op.kernel_name(M) == "ExactKernel"
+    Y = op(torch.from_numpy(A).to(cuda)).cpu().numpy()
+    op.release()
+    group = -(-K // 64) * 2 * 256  # words of 64 columns, which follow each other in the copy
+    last = (-(-N // 256) * 4 * group - 2**32) // group * 64
+    cols = [0, 1, last - 1, last, last + 64, last + 128, 131071, N - 1]
+    y64 = orc.matmul_nbits_f64(A, B[cols].cpu().numpy(), S[cols].cpu().numpy(), None, K, len(cols), bs)
+    del B, S
+    torch.cuda.empty_cache()
+    assert orc.normwise_max_error(Y[:, cols], y64) <= TOL
