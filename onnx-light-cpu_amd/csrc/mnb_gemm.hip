@@ -1580,15 +1580,16 @@ __global__ __launch_bounds__(256) void RelayoutBKernel(const uint8_t *__restrict
                                                        uint32_t *__restrict__ Bp, int64_t N,
                                                        int64_t row_bytes, int64_t T,
                                                        int64_t words) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= words) return;
-  const int j = static_cast<int>(idx & 3);
-  const int l = static_cast<int>((idx >> 2) & 63);
-  const int64_t gs = idx >> 8;
-  const int64_t s = gs % T, g = gs / T;
-  const int64_t n = 64 * g + 16 * j + (l & 15);
-  Bp[idx] = n < N ? *reinterpret_cast<const uint32_t *>(B + n * row_bytes + 16 * s + 4 * (l >> 4))
-                  : 0u;
+  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < words;
+       idx += static_cast<int64_t>(gridDim.x) * 256) {
+    const int j = static_cast<int>(idx & 3);
+    const int l = static_cast<int>((idx >> 2) & 63);
+    const int64_t gs = idx >> 8;
+    const int64_t s = gs % T, g = gs / T;
+    const int64_t n = 64 * g + 16 * j + (l & 15);
+    Bp[idx] = n < N ? *reinterpret_cast<const uint32_t *>(B + n * row_bytes + 16 * s + 4 * (l >> 4))
+                    : 0u;
+  }
 }
 
 __global__ __launch_bounds__(256) void RelayoutSKernel(const float *__restrict__ S,
@@ -1597,20 +1598,21 @@ __global__ __launch_bounds__(256) void RelayoutSKernel(const float *__restrict__
                                                        uint32_t *__restrict__ Sp, int64_t N,
                                                        int64_t nb, int64_t zp_row_bytes,
                                                        int64_t words) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= words) return;
-  const int j = static_cast<int>(idx & 3);
-  const int c = static_cast<int>((idx >> 2) & 15);
-  const int64_t gb = idx >> 6;
-  const int64_t b = gb % nb, g = gb / nb;
-  const int64_t n = 64 * g + 16 * j + c;
-  uint32_t v = (8u << 16) | (8u << 28);  // rows past N: scale 0
-  if (n < N) {
-    const _Float16 h = static_cast<_Float16>(__builtin_amdgcn_ldexpf(S[n * nb + b], col_exp[n]));
-    const uint32_t z = Z != nullptr ? (Z[n * zp_row_bytes + (b >> 1)] >> (4 * (b & 1))) & 0xFu : 8u;
-    v = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) | (z << 16) | (z << 28);
+  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < words;
+       idx += static_cast<int64_t>(gridDim.x) * 256) {
+    const int j = static_cast<int>(idx & 3);
+    const int c = static_cast<int>((idx >> 2) & 15);
+    const int64_t gb = idx >> 6;
+    const int64_t b = gb % nb, g = gb / nb;
+    const int64_t n = 64 * g + 16 * j + c;
+    uint32_t v = (8u << 16) | (8u << 28);  // rows past N: scale 0
+    if (n < N) {
+      const _Float16 h = static_cast<_Float16>(__builtin_amdgcn_ldexpf(S[n * nb + b], col_exp[n]));
+      const uint32_t z = Z != nullptr ? (Z[n * zp_row_bytes + (b >> 1)] >> (4 * (b & 1))) & 0xFu : 8u;
+      v = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) | (z << 16) | (z << 28);
+    }
+    Sp[idx] = v;
   }
-  Sp[idx] = v;
 }
 
 bool PrefillSupportsShape(const WeightView &w) {
@@ -1843,13 +1845,12 @@ hipError_t LaunchPrefillRelayout(const WeightView &w, uint8_t *Bp, uint8_t *Sp, 
   const size_t bp_bytes = PrefillLayoutBytes(w, &sp_bytes);
   const int64_t T = w.K / 32;
   const int64_t bw = static_cast<int64_t>(bp_bytes / 4), sw = static_cast<int64_t>(sp_bytes / 4);
-  hipLaunchKernelGGL(RelayoutBKernel, dim3(static_cast<unsigned>((bw + 255) / 256)), dim3(256), 0,
-                     s, w.B, reinterpret_cast<uint32_t *>(Bp), w.N, w.row_bytes, T, bw);
+  hipLaunchKernelGGL(RelayoutBKernel, StrideGrid(bw), dim3(256), 0, s, w.B,
+                     reinterpret_cast<uint32_t *>(Bp), w.N, w.row_bytes, T, bw);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(RelayoutSKernel, dim3(static_cast<unsigned>((sw + 255) / 256)), dim3(256), 0,
-                     s, w.scales, w.zp, w.col_exp, reinterpret_cast<uint32_t *>(Sp), w.N, w.nb,
-                     w.zp_row_bytes, sw);
+  hipLaunchKernelGGL(RelayoutSKernel, StrideGrid(sw), dim3(256), 0, s, w.scales, w.zp,
+                     w.col_exp, reinterpret_cast<uint32_t *>(Sp), w.N, w.nb, w.zp_row_bytes, sw);
   return hipGetLastError();
 }
 

@@ -250,3 +250,34 @@ def test_small_m_decode_four_units_per_wavefront(pkg, orc, cuda, K, N, bs, zp, o
             assert err <= GEMV_TOL and err_old <= GEMV_TOL
     finally:
         op.release()
+
+
+def test_weights_of_18_gb(pkg, orc, cuda):
+    """18 GB of weights: their re-laid copy has more than 2^32 words, and one
+    launch has fewer threads than that. Columns from its start, its end and both
+    sides of the word where the launch's threads would end."""
+    import torch
+    K, N, bs = 131072, 270000, 256
+    nb = K // bs
+    if torch.cuda.mem_get_info(cuda)[0] < 45 << 30:
+        pytest.skip("less than 45 GiB of device memory free")
+    gen = torch.Generator(device=cuda).manual_seed(7)
+    B = torch.randint(0, 256, (N, nb, bs // 2), dtype=torch.uint8, device=cuda, generator=gen)
+    S = torch.rand((N, nb), device=cuda, generator=gen) * 0.015 + 0.005
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare_device(B, S)
+    group = K // 32 * 256  # words of 64 columns, which follow each other in the copy
+    last = (-(-N // 256) * 4 * group - 2**32) // group * 64
+    cols = [0, 1, last - 1, last, last + 64, last + 128, 131071, N - 1]
+    for M, tol in ((3, GEMV_TOL), (256, GEMM_TOL)):
+        print(f"case large 18 GB K={K} N={N} bs={bs} M={M} kernel={op.kernel_name(M)}", flush=True)
+        assert op.kernel_name(M) in ("DecodeFragKernel", "PrefillKernel", "WideKernel")
+        A = pkg.workloads.make_activations(M, K, 1.0, M)
+        Y = op(torch.from_numpy(A).to(cuda)).cpu().numpy()[:, cols]
+        y64 = orc.matmul_nbits_f64(A, B[cols].cpu().numpy(), S[cols].cpu().numpy(), None, K,
+                                   len(cols), bs)
+        err = orc.normwise_max_error(Y, y64) if M <= 16 else orc.l2_rel_error(Y, y64)
+        print(f"  error vs fp64 {err:.2e}")
+        assert err <= tol
+    op.release()
+    del B, S
+    torch.cuda.empty_cache()
