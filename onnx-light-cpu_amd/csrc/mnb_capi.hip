@@ -213,32 +213,34 @@ int DerivePlanConstants(mnb_plan *p) {
       FillView(p);
     }
   } else if (mnb::ExactRaggedLayoutWanted(p->view)) {
-    // K that 64-k tiles do not divide: the exact GEMM's layout alone.
+    // K that 64-k tiles do not divide: the exact GEMM's layout alone. Where its
+    // memory is not to be had, or with scales that it does not take,
+    // GenericKernel serves the plan.
     size_t zd_bytes = 0;
     const size_t bp_bytes = mnb::ExactRaggedLayoutBytes(p->view);
     const size_t sd_bytes = mnb::DecodeFragScaleBytes(p->view, &zd_bytes);
+    auto without = [&]() {
+      if (p->dSd) (void)hipFree(p->dSd);
+      if (p->dBp) (void)hipFree(p->dBp);
+      if (p->dZd) (void)hipFree(p->dZd);
+      p->dSd = nullptr;
+      p->dBp = nullptr;
+      p->dZd = nullptr;
+      if (e != hipSuccess) (void)hipGetLastError();  // the failed allocation's
+      return MNB_OK;
+    };
     e = hipMalloc(reinterpret_cast<void **>(&p->dSd), sd_bytes);
-    if (e != hipSuccess) {
-      SetLastError("hipMalloc", e);
-      return MNB_ERR_ALLOC;
-    }
+    if (e != hipSuccess) return without();
     bool scales_ok = false;  // dSd holds at least 64 words
     e = mnb::ExactRaggedScalesOk(p->view, reinterpret_cast<uint32_t *>(p->dSd), &scales_ok);
     if (e != hipSuccess) {
       SetLastError("plan constants", e);
       return MNB_ERR_HIP;
     }
-    if (!scales_ok) {  // GenericKernel serves the plan
-      (void)hipFree(p->dSd);
-      p->dSd = nullptr;
-      return MNB_OK;
-    }
+    if (!scales_ok) return without();
     e = hipMalloc(reinterpret_cast<void **>(&p->dBp), bp_bytes);
     if (e == hipSuccess && zd_bytes > 0) e = hipMalloc(reinterpret_cast<void **>(&p->dZd), zd_bytes);
-    if (e != hipSuccess) {
-      SetLastError("hipMalloc", e);
-      return MNB_ERR_ALLOC;
-    }
+    if (e != hipSuccess) return without();
     e = mnb::LaunchExactRaggedRelayout(p->view, p->dBp, nullptr);
     if (e == hipSuccess) e = mnb::LaunchDecodeFragRelayout(p->view, p->dSd, p->dZd, nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);

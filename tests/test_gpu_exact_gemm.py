@@ -364,3 +364,28 @@ def test_ragged_weights_of_18_gb(pkg, orc, cuda):
     del B, S
     torch.cuda.empty_cache()
     assert orc.normwise_max_error(Y[:, cols], y64) <= TOL
+
+
+def test_ragged_weights_that_fit_once(pkg, orc, cuda):
+    """Weights of 55% of the free device memory: no room for the exact GEMM's
+    copy. The plan is created all the same and the generic kernel serves it."""
+    import torch
+    torch.cuda.empty_cache()
+    K, bs = 131073, 256
+    nb = -(-K // bs)
+    N = int(torch.cuda.mem_get_info(cuda)[0] * 0.55) // (nb * bs // 2)
+    if N >= 1 << 22:
+        pytest.skip("more device memory than this width fills")
+    B = torch.empty((N, nb, bs // 2), dtype=torch.uint8, device=cuda)
+    S = torch.full((N, nb), 0.01, device=cuda)
+    print(f"case ragged fits once K={K} N={N} bs={bs} {B.numel()} bytes", flush=True)
+    op = pkg.MatMulNBits(K, N, 4, bs).prepare_device(B, S)
+    assert op.kernel_name(1) == "GenericKernel"
+    A = pkg.workloads.make_activations(1, K, 1.0, 8)
+    Y = op(torch.from_numpy(A).to(cuda)).cpu().numpy()
+    op.release()
+    cols = [0, N // 2, N - 1]
+    y64 = orc.matmul_nbits_f64(A, B[cols].cpu().numpy(), S[cols].cpu().numpy(), None, K, len(cols), bs)
+    del B, S
+    torch.cuda.empty_cache()
+    assert np.abs(Y[:, cols] - y64).max() <= TOL * 8 * 0.01 * np.abs(A).sum()
