@@ -17,7 +17,7 @@ from __future__ import annotations
 import ctypes
 import os
 import pathlib
-import threading
+from threading import get_ident
 
 import numpy as np
 
@@ -138,10 +138,16 @@ def _dev_ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+_C = None  # torch._C
+
+
 def _raw_stream(device):
     """The handle of the device's current stream."""
-    import torch
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    global _C
+    if _C is None:
+        import torch
+        _C = torch._C
+    return _C._cuda_getCurrentRawStream(device.index)
 
 
 class MatMulNBits:
@@ -357,12 +363,14 @@ class MatMulNBits:
         # Up to 8 are kept, the oldest is dropped. An allocation per call took 2.5 us
         # longer (K = 2500, N = 5001, 333 rows 47.5 -> 50.0 us: its memory and the
         # output's change places in the caches). A captured call has the graph's own.
-        import torch
-        if torch.cuda.is_current_stream_capturing():
+        raw = _raw_stream(device)
+        if raw != 0 and _C._cuda_isCurrentStreamCapturing():  # not the default stream
+            import torch
             return torch.empty(need, dtype=torch.uint8, device=device)
-        key = (threading.get_ident(), _raw_stream(device), device)
+        key = (get_ident(), raw, device.index)
         work = self._works.get(key)
         if work is None or work.numel() < need:
+            import torch
             for old in list(self._works)[:-7]:
                 self._works.pop(old, None)
             work = self._works[key] = torch.empty(need, dtype=torch.uint8, device=device)

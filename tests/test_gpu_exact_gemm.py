@@ -339,6 +339,23 @@ def test_ragged_calls_on_two_streams(pkg, cuda, explicit):
         assert all(torch.equal(o.cpu(), w) for o in out)
 
 
+def test_gate_up_generic_path(pkg, orc, cuda):
+    """The generic path chosen by the caller on a gate/up plan: its scratch sum is
+    the one workspace that it needs."""
+    import torch
+    K, I, bs, M = 1000, 100, 32, 20
+    p = pkg.workloads.Projection("gu", K, I, bs, True)
+    W = [pkg.workloads.make_weights(p, s) for s in (81, 82)]
+    gu = pkg.GateUpSiLU(K, I, 4, bs).prepare(*W[0], *W[1])
+    A = pkg.workloads.make_activations(M, K, 1.0, 83)
+    dA = torch.from_numpy(A).to(cuda)
+    print(f"case gate/up generic K={K} I={I} M={M}", flush=True)
+    H = gu(dA, path=pkg.PATH_GENERIC, stream=torch.cuda.current_stream()).cpu().numpy()
+    gu.release()
+    h64 = orc.gate_up_silu_f64(A, *W[0], *W[1], K, I, bs)
+    assert orc.normwise_max_error(H, h64) <= 4 * TOL
+
+
 def test_ragged_weights_of_18_gb(pkg, orc, cuda):
     """18 GB of weights: their re-laid copy has more than 2^32 words, and one
     launch has fewer threads than that. Columns from its start, its end and both
