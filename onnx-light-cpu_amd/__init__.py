@@ -363,7 +363,12 @@ class MatMulNBits:
         # Up to 8 are kept, the oldest is dropped. An allocation per call took 2.5 us
         # longer (K = 2500, N = 5001, 333 rows 47.5 -> 50.0 us: its memory and the
         # output's change places in the caches). A captured call has the graph's own.
-        raw = _raw_stream(device)
+        try:
+            raw = _raw_stream(device)
+        except TypeError:  # a name, or a device without its index
+            import torch
+            device = torch.empty(0, device=device).device
+            raw = _raw_stream(device)
         if raw != 0 and _C._cuda_isCurrentStreamCapturing():  # not the default stream
             import torch
             return torch.empty(need, dtype=torch.uint8, device=device)

@@ -324,6 +324,8 @@ def test_ragged_calls_on_two_streams(pkg, cuda, explicit):
             works.append(op.workspace(M, cuda))
     assert len({w.data_ptr() for w in works}) == 9 and len(op._works) == 8
     del works
+    names = [op.workspace(M, d) for d in (cuda, "cuda:0", "cuda", torch.device("cuda"))]
+    assert len({w.data_ptr() for w in names}) == 1  # one stream, one workspace
     outs = [[torch.empty(M, N, device=cuda) for _ in range(16)] for _ in As]
     torch.cuda.synchronize()
     for i in range(16):
