@@ -365,7 +365,7 @@ class MatMulNBits:
         # output's change places in the caches). A captured call has the graph's own.
         try:
             raw = _raw_stream(device)
-        except TypeError:  # a name, or a device without its index
+        except (TypeError, RuntimeError):  # a name, or a device without its index
             import torch
             device = torch.empty(0, device=device).device
             raw = _raw_stream(device)
